@@ -104,6 +104,11 @@ struct kahan {
     c = (t - s) - y;
     s = t;
   }
+  // Another accumulator's sum, its lost low-order part with it.
+  __device__ __forceinline__ void merge(T os, T oc) {
+    add(os);
+    add(-oc);
+  }
 };
 
 }  // namespace ptyrs

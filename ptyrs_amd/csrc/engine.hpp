@@ -824,7 +824,7 @@ class Engine : public EngineBase {
     pden_part_.ensure(sizeof(T) * size_t(nstack) * nchunk * n);
     pnum_.ensure(sizeof(cplx<T>) * M_ * n);
     pden_.ensure(sizeof(T) * n);
-    pmaxpart_.ensure(sizeof(T) * ((n + THREADS - 1) / THREADS));
+    pmaxpart_.ensure(sizeof(T) * ((n + REDUCE_PX - 1) / REDUCE_PX));
     pmax2_.ensure(sizeof(T) * 2);
     abs_part_.ensure(sizeof(double) * 2 * kAbsBlocks);
     probe_terms();
@@ -1048,8 +1048,7 @@ class Engine : public EngineBase {
     const int nt = ntiles();
     const cplx<T>* wall = wall_.as<cplx<T>>();
     run(K_BIN, [&] {
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
+      bin_tiles(corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
                          int(nframe_), list_all_.as<int>(), count_all_.as<int>(),
                          (const T*)nullptr, M_, int(nyo_), int(nxo_), D_.as<T>(),
                          tilemax_.as<T>(), wall);
@@ -1059,8 +1058,7 @@ class Engine : public EngineBase {
                          tilemax_.as<T>(), nt, pmax_.as<T>());
     });
     run(K_OBJ_UPDATE, [&] {
-      hipLaunchKernelGGL((k_obj_blend<T, false>), dim3(nt), dim3(THREADS), 0, stream_,
-                         O_.as<cplx<T>>(), wall, D_.as<T>(),
+      obj_blend<false>(O_.as<cplx<T>>(), wall, D_.as<T>(),
                          Carried<T, false>{carried_.as<cplx<T>>()}, N, M_, corner_.as<int2>(),
                          iota_.as<int>(), list_all_.as<int>(), count_all_.as<int>(),
                          int(nframe_), int(nyo_), int(nxo_), ntx_, pmax_.as<T>(), T(inertia), 1);
@@ -1455,7 +1453,7 @@ class Engine : public EngineBase {
     pden_part_.ensure(sizeof(T) * size_t(nstack) * nchunk * n);
     pnum_.ensure(sizeof(cplx<T>) * M_ * n);
     pden_.ensure(sizeof(T) * n);
-    pmaxpart_.ensure(sizeof(T) * ((n + THREADS - 1) / THREADS));
+    pmaxpart_.ensure(sizeof(T) * ((n + REDUCE_PX - 1) / REDUCE_PX));
     abs_part_.ensure(sizeof(double) * 2 * kAbsBlocks);
     cg_part_.ensure(sizeof(double) * 2 * kAbsBlocks);
     cg_sums_.ensure(sizeof(double) * 2);
@@ -1471,8 +1469,7 @@ class Engine : public EngineBase {
     balance(1.0, hist_.as<double>() + 3);
     if (uo) {
       run(K_BIN, [&] {
-        hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
+        bin_tiles(corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
                            int(nframe_), list_all_.as<int>(), count_all_.as<int>(),
                            (const T*)nullptr, M_, int(nyo_), int(nxo_), (T*)nullptr,
                            tilemax_.as<T>(),
@@ -1515,17 +1512,17 @@ class Engine : public EngineBase {
       }
       if (uo) {
         run(K_OBJ_UPDATE, [&] {
-          hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                             gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), carried_.as<cplx<T>>(), N,
+          obj_dir(gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), carried_.as<cplx<T>>(), N,
                              M_, corner_.as<int2>(), iota_.as<int>(), list_all_.as<int>(),
                              count_all_.as<int>(), int(nframe_), int(nyo_), int(nxo_), ntx_,
                              (const T*)nullptr, (const T*)nullptr);
         });
       }
       if (up) {
-        const int nblk = (n + THREADS - 1) / THREADS;
+        const int nblk = (n + REDUCE_PX - 1) / REDUCE_PX;
         run(K_PROBE, [&] {
-          hipLaunchKernelGGL(k_probe_reduce<T>, dim3(nblk), dim3(THREADS), 0, stream_,
+          hipLaunchKernelGGL(k_probe_reduce<T>, dim3(nblk, M_ + 1), dim3(REDUCE_THREADS), 0,
+                             stream_,
                              pnum_part_.as<cplx<T>>(), pden_part_.as<T>(), nstack * nchunk, n,
                              M_, gP_.as<cplx<T>>(), pden_.as<T>(), pmaxpart_.as<T>());
         });
@@ -1655,8 +1652,7 @@ class Engine : public EngineBase {
     balance(1.0, hist_.as<double>() + 3);
     if (uo) {
       run(K_BIN, [&] {
-        hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
+        bin_tiles(corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
                            int(nframe_), list_all_.as<int>(), count_all_.as<int>(),
                            (const T*)nullptr, M_, int(nyo_), int(nxo_), (T*)nullptr,
                            tilemax_.as<T>(), (const cplx<T>*)nullptr);
@@ -1760,8 +1756,7 @@ class Engine : public EngineBase {
       }
       if (uo) {
         run(K_OBJ_UPDATE, [&] {
-          hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                             gO_.as<cplx<T>>(), (const cplx<T>*)wall, carried_.as<cplx<T>>(),
+          obj_dir(gO_.as<cplx<T>>(), (const cplx<T>*)wall, carried_.as<cplx<T>>(),
                              N, M_, corner_.as<int2>(), iota_.as<int>(), list_all_.as<int>(),
                              count_all_.as<int>(), int(nframe_), int(nyo_), int(nxo_), ntx_,
                              (const T*)nullptr, (const T*)nullptr, 1, (const cplx<T>*)nullptr,
@@ -2993,8 +2988,7 @@ class Engine : public EngineBase {
     const bool refine = pos_refine_;
     const double2* offs = offs_.as<double2>();
     run(K_BIN, [&] {
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+      bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                          lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                          (T*)nullptr, tilemax_.as<T>(), (const cplx<T>*)nullptr);
     });
@@ -3013,8 +3007,7 @@ class Engine : public EngineBase {
                          chunk, 0, dP_.as<cplx<T>>(), tw_.as<cplx<T>>(), 0);
     });
     run(K_OBJ_DIR, [&] {
-      hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         bh_gO_.as<cplx<T>>(), (const cplx<T>*)w, psi_.as<cplx<T>>(), N, M_,
+      obj_dir(bh_gO_.as<cplx<T>>(), (const cplx<T>*)w, psi_.as<cplx<T>>(), N, M_,
                          corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                          int(nyo_), int(nxo_), ntx_, (const T*)nullptr, (const T*)nullptr, 1);
     });
@@ -3118,8 +3111,7 @@ class Engine : public EngineBase {
         fo_slice_windows(ord, nb);
         return;
       }
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+      bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                          lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                          (T*)nullptr, tilemax_.as<T>(), (const cplx<T>*)nullptr);
     });
@@ -3157,8 +3149,7 @@ class Engine : public EngineBase {
           fo_add_placed<AS_PLAIN>(bh_gO_.as<cplx<T>>() + s * no1, 1.0);
           return;
         }
-        hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           bh_gO_.as<cplx<T>>() + s * no1, in.first, (const cplx<T>*)chi, N, M_,
+        obj_dir(bh_gO_.as<cplx<T>>() + s * no1, in.first, (const cplx<T>*)chi, N, M_,
                            corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                            int(nyo_), int(nxo_), ntx_, (const T*)nullptr, (const T*)nullptr,
                            in.second, qs, 0);
@@ -3344,8 +3335,8 @@ class Engine : public EngineBase {
       fo_add_placed<AS_PLAIN>(bh_gO_.p, 1.0);
     });
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_probe_mean<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                         bh_gP_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, 1);
+      hipLaunchKernelGGL(k_probe_mean<T>, dim3(chunk_blocks(total, nchunk)), dim3(THREADS), 0,
+                         stream_, bh_gP_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, 1);
     });
     const int ndots =
         int(std::min<size_t>(kBhDotBlocks, (no + np + THREADS - 1) / THREADS));
@@ -3476,8 +3467,7 @@ class Engine : public EngineBase {
     const size_t no = nyo_ * nxo_, np = nprobe_ * n;
     const int total = int(np);
     run(K_BIN, [&] {
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+      bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                          lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                          (T*)nullptr, tilemax_.as<T>(), (const cplx<T>*)nullptr);
     });
@@ -3494,14 +3484,13 @@ class Engine : public EngineBase {
                          chunk, 1, dP_.as<cplx<T>>(), tw_.as<cplx<T>>(), 0);
     });
     run(K_OBJ_DIR, [&] {
-      hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         bh_gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
+      obj_dir(bh_gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
                          corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                          int(nyo_), int(nxo_), ntx_, (const T*)nullptr, (const T*)nullptr);
     });
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_probe_mean<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                         bh_gP_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, 1);
+      hipLaunchKernelGGL(k_probe_mean<T>, dim3(chunk_blocks(total, nchunk)), dim3(THREADS), 0,
+                         stream_, bh_gP_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, 1);
     });
     const int ndots =
         int(std::min<size_t>(kBhDotBlocks, (no + np + THREADS - 1) / THREADS));
@@ -3563,17 +3552,19 @@ class Engine : public EngineBase {
       const int nb = std::min(step, int(nframe_) - f0);
       const int* ord = iota_.as<int>() + f0;
       run(K_BIN, [&] {
-        hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           corner_.as<int2>(), ord, nb, N, ntx_, step, list_all_.as<int>(),
+        bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, step, list_all_.as<int>(),
                            count_all_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                            (T*)nullptr, tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
       });
       run(K_OTHER, [&] {
-        hipLaunchKernelGGL(k_illumination<T>, dim3(nt), dim3(THREADS), 0, stream_,
+        split_tiles([&](auto sp) {
+          constexpr int SP = decltype(sp)::value;
+          hipLaunchKernelGGL((k_illumination<T, SP>), dim3(nt), dim3(THREADS * SP), 0, stream_,
                            illum_.as<T>(), P_.as<cplx<T>>(), N, M_, corner_.as<int2>(), ord,
                            list_all_.as<int>(), count_all_.as<int>(), step, int(nyo_),
                            int(nxo_), ntx_);
+        });
       });
     }
     const double init = max_frame_total_ / (4.0 * double(n) * scale_);
@@ -3590,8 +3581,7 @@ class Engine : public EngineBase {
     const int nt = ntiles();
     const bool gauss = p.cost == PTYRS_AMPLITUDE;
     run(K_BIN, [&] {
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+      bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                          lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                          (T*)nullptr, tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
@@ -3634,8 +3624,7 @@ class Engine : public EngineBase {
                          chunk, 1, dP_.as<cplx<T>>(), tw_.as<cplx<T>>());
     });
     run(K_OBJ_DIR, [&] {
-      hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
+      obj_dir(dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
                          corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                          int(nyo_), int(nxo_), ntx_, pre_.as<T>(), floor_.as<T>());
     });
@@ -3644,8 +3633,8 @@ class Engine : public EngineBase {
     // λ0 = 1.2e-7·k/n per pixel and mode (ptyrs/src/engine/lsqml.rs:31-33), summed over both.
     const double lam = 1.2e-7 * scale_ * double(M_);
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_probe_mean<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                         dPm_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, nb);
+      hipLaunchKernelGGL(k_probe_mean<T>, dim3(chunk_blocks(total, nchunk)), dim3(THREADS), 0,
+                         stream_, dPm_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, nb);
     });
     run(K_DOTS, [&] {
       hipLaunchKernelGGL(k_lsqml_dots<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
@@ -3703,8 +3692,7 @@ class Engine : public EngineBase {
       const int K = nb * M_;
       const int acc = f0 > 0;
       run(K_BIN, [&] {
-        hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+        bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                            lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                            (T*)nullptr, tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
@@ -3721,8 +3709,7 @@ class Engine : public EngineBase {
         const auto in = wave(s, wv);
         const cplx<T>* qs = s + 1 == S ? q_.as<cplx<T>>() : nullptr;
         run(K_OBJ_UPDATE, [&] {
-          hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                             slice_dir(s), in.first, (const cplx<T>*)chi, N, M_,
+          obj_dir(slice_dir(s), in.first, (const cplx<T>*)chi, N, M_,
                              corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(),
                              int(cap_), int(nyo_), int(nxo_), ntx_, (const T*)nullptr,
                              (const T*)nullptr, in.second, qs, 0, acc);
@@ -3819,8 +3806,7 @@ class Engine : public EngineBase {
         fo_slice_windows(ord, nb);
         return;
       }
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+      bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                          lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                          (T*)nullptr, tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
@@ -3882,8 +3868,7 @@ class Engine : public EngineBase {
                              (const T*)floor_.as<T>(), nol);
           return;
         }
-        hipLaunchKernelGGL(k_lsqml_obj_dir<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           slice_dir(s), in.first, (const cplx<T>*)chi, N, M_, corner_.as<int2>(),
+        obj_dir(slice_dir(s), in.first, (const cplx<T>*)chi, N, M_, corner_.as<int2>(),
                            ord, list_.as<int>(), lcount_.as<int>(), int(cap_), int(nyo_),
                            int(nxo_), ntx_, pre_.as<T>(), floor_.as<T>(), in.second, qs, qf);
       });
@@ -4051,8 +4036,7 @@ class Engine : public EngineBase {
     const int nt = ntiles();
     run(K_BIN, [&] {
       norm2_planes();
-      hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                         corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
+      bin_tiles(corner_.as<int2>(), iota_.as<int>(), int(nframe_), N, ntx_,
                          int(nframe_), list_all_.as<int>(), count_all_.as<int>(),
                          (const T*)W2_.as<T>(), M_, int(nyo_), int(nxo_), D_.as<T>(),
                          tilemax_.as<T>(),
@@ -4063,8 +4047,7 @@ class Engine : public EngineBase {
                          tilemax_.as<T>(), nt, pmax_.as<T>());
     });
     run(K_OBJ_UPDATE, [&] {
-      hipLaunchKernelGGL((k_obj_blend<T, H>), dim3(nt), dim3(THREADS), 0, stream_,
-                         O_.as<cplx<T>>(), Wt_.as<cplx<T>>(), D_.as<T>(), cw, N, M_,
+      obj_blend<H>(O_.as<cplx<T>>(), Wt_.as<cplx<T>>(), D_.as<T>(), cw, N, M_,
                          corner_.as<int2>(), iota_.as<int>(),
                          list_all_.as<int>(), count_all_.as<int>(), int(nframe_), int(nyo_),
                          int(nxo_), ntx_, pmax_.as<T>(), T(inertia));
@@ -4092,10 +4075,11 @@ class Engine : public EngineBase {
   }
 
   void probe_blend(int tot_chunks, double inertia) {
-    const int nblk = (n + THREADS - 1) / THREADS;
+    const int nblk = (n + REDUCE_PX - 1) / REDUCE_PX;
     const int total = int(nprobe_ * n);
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_probe_reduce<T>, dim3(nblk), dim3(THREADS), 0, stream_,
+      hipLaunchKernelGGL(k_probe_reduce<T>, dim3(nblk, M_ + 1), dim3(REDUCE_THREADS), 0,
+                             stream_,
                          pnum_part_.as<cplx<T>>(), pden_part_.as<T>(), tot_chunks, n, M_,
                          pnum_.as<cplx<T>>(), pden_.as<T>(), pmaxpart_.as<T>());
       hipLaunchKernelGGL(k_max_reduce<T>, dim3(1), dim3(MAX_THREADS), 0, stream_,
@@ -4154,6 +4138,65 @@ class Engine : public EngineBase {
   }
 
   int ntiles() const { return ntx_ * nty_; }
+  // The tile kernels' split (SP of them share a tile's views; kernels.hpp): by the tile count.
+  template <typename F>
+  void split_tiles(F&& f) {
+    if (ntiles() < kSplitTiles)
+      f(std::integral_constant<int, 4>{});
+    else
+      f(std::integral_constant<int, 1>{});
+  }
+  // Modes whose loads the tile gathers issue together: 1, 2 or (3 and more) 4.
+  template <typename F>
+  void mode_chunk(F&& f) {
+    if (M_ == 1)
+      f(std::integral_constant<int, 1>{});
+    else if (M_ == 2)
+      f(std::integral_constant<int, 2>{});
+    else
+      f(std::integral_constant<int, 4>{});
+  }
+  // Workgroups of k_probe_apply and k_probe_mean.
+  static unsigned chunk_blocks(int total, int nchunk) {
+    const int px = chunk_px(nchunk, THREADS);
+    return unsigned((total + px - 1) / px);
+  }
+  void bin_tiles(const int2* corner, const int* ord, int nb, int side, int ntx, int cap, int* list,
+                 int* count, const T* W2, int M, int nyo, int nxo, T* D, T* tilemax,
+                 const cplx<T>* Wv) {
+    split_tiles([&](auto sp) {
+      constexpr int SP = decltype(sp)::value;
+      hipLaunchKernelGGL((k_bin_tiles<T, SP>), dim3(ntiles()), dim3(THREADS * SP), 0, stream_,
+                         corner, ord, nb, side, ntx, cap, list, count, W2, M, nyo, nxo, D,
+                         tilemax, Wv);
+    });
+  }
+  void obj_dir(cplx<T>* dO, const cplx<T>* Wt, const cplx<T>* chi, int side, int M,
+               const int2* corner, const int* ord, const int* list, const int* count, int cap,
+               int nyo, int nxo, int ntx, const T* pre, const T* floor, int per_view = 0,
+               const cplx<T>* q = nullptr, int q_frame = 0, int accumulate = 0) {
+    split_tiles([&](auto sp) {
+      mode_chunk([&](auto mm) {
+        constexpr int SP = decltype(sp)::value, MM = decltype(mm)::value;
+        hipLaunchKernelGGL((k_lsqml_obj_dir<T, SP, MM>), dim3(ntiles()), dim3(THREADS * SP), 0,
+                           stream_, dO, Wt, chi, side, M, corner, ord, list, count, cap, nyo,
+                           nxo, ntx, pre, floor, per_view, q, q_frame, accumulate);
+      });
+    });
+  }
+  template <bool H>
+  void obj_blend(cplx<T>* O, const cplx<T>* Wt, const T* D, Carried<T, H> cw, int side, int M,
+                 const int2* corner, const int* ord, const int* list, const int* count, int cap,
+                 int nyo, int nxo, int ntx, const T* nmax, T inertia, int w_view = 0) {
+    split_tiles([&](auto sp) {
+      mode_chunk([&](auto mm) {
+        constexpr int SP = decltype(sp)::value, MM = decltype(mm)::value;
+        hipLaunchKernelGGL((k_obj_blend<T, H, SP, MM>), dim3(ntiles()), dim3(THREADS * SP), 0,
+                           stream_, O, Wt, D, cw, side, M, corner, ord, list, count, cap, nyo,
+                           nxo, ntx, nmax, inertia, w_view);
+      });
+    });
+  }
 
   // Pass C chunking: enough workgroups to fill the chip, few partial probe sums.
   int chunk_of(int nb) const {
@@ -4402,8 +4445,7 @@ class Engine : public EngineBase {
       // W2_ holds |W_m|² of the batch-start probe terms (rpie_begin, then each batch's
       // k_rpie_updates; without probe updates the probe does not change).
       run(K_BIN, [&] {
-        hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+        bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                            lcount_.as<int>(), (const T*)W2_.as<T>(), M_, int(nyo_), int(nxo_),
                            D_.as<T>(), tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
@@ -4434,29 +4476,36 @@ class Engine : public EngineBase {
     if (upd_obj && upd_probe) {
       const int total = int(nprobe_ * n);
       run(K_OBJ_UPDATE, [&] {
-        hipLaunchKernelGGL(k_rpie_updates<T>, dim3(nt + (total + THREADS - 1) / THREADS),
-                           dim3(THREADS), 0, stream_, O_.as<cplx<T>>(),
+        split_tiles([&](auto sp) {
+          constexpr int SP = decltype(sp)::value, BT = THREADS * SP;
+          const int px = chunk_px(nchunk, BT);
+          hipLaunchKernelGGL((k_rpie_updates<T, SP>), dim3(nt + (total + px - 1) / px), dim3(BT), 0,
+                           stream_, O_.as<cplx<T>>(),
                            (const cplx<T>*)psi_.as<cplx<T>>(), N, M_, corner_.as<int2>(), ord,
                            list_.as<int>(), lcount_.as<int>(), int(cap_), int(nyo_), int(nxo_),
                            ntx_, T(p.obj_step), nt, P_.as<cplx<T>>(), Wt_.as<cplx<T>>(),
                            q_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total,
                            T(p.probe_step / nb), W2_.as<T>());
+        });
       });
       return;
     }
     if (upd_obj) {
       run(K_OBJ_UPDATE, [&] {
-        hipLaunchKernelGGL(k_obj_update_rpie_sum<T>, dim3(nt), dim3(THREADS), 0, stream_,
+        split_tiles([&](auto sp) {
+          constexpr int SP = decltype(sp)::value;
+          hipLaunchKernelGGL((k_obj_update_rpie_sum<T, SP>), dim3(nt), dim3(THREADS * SP), 0, stream_,
                            O_.as<cplx<T>>(), (const cplx<T>*)psi_.as<cplx<T>>(), N, M_,
                            corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(),
                            int(cap_), int(nyo_), int(nxo_), ntx_, T(p.obj_step));
+        });
       });
     }
     if (upd_probe) {
       const int total = int(nprobe_ * n);
       run(K_PROBE, [&] {
-        hipLaunchKernelGGL(k_probe_apply<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                           P_.as<cplx<T>>(), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
+        hipLaunchKernelGGL(k_probe_apply<T>, dim3(chunk_blocks(total, nchunk)), dim3(THREADS), 0,
+                           stream_, P_.as<cplx<T>>(), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
                            dP_.as<cplx<T>>(), nchunk, n, total, T(p.probe_step / nb));
       });
     }
@@ -4479,8 +4528,7 @@ class Engine : public EngineBase {
     const cplx<T>* W = inc0_.as<cplx<T>>();
     if (upd_obj) {
       run(K_BIN, [&] {
-        hipLaunchKernelGGL(k_bin_tiles<T>, dim3(nt), dim3(THREADS), 0, stream_,
-                           corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
+        bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                            lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
                            D_.as<T>(), tilemax_.as<T>(), W);
       });
@@ -4509,10 +4557,13 @@ class Engine : public EngineBase {
     if (pos_refine_) position_sums(0, W, nullptr, 0, ord, nb, chi0);
     if (upd_obj) {
       run(K_OBJ_UPDATE, [&] {
-        hipLaunchKernelGGL(k_obj_update_rpie_sum<T>, dim3(nt), dim3(THREADS), 0, stream_,
+        split_tiles([&](auto sp) {
+          constexpr int SP = decltype(sp)::value;
+          hipLaunchKernelGGL((k_obj_update_rpie_sum<T, SP>), dim3(nt), dim3(THREADS * SP), 0, stream_,
                            O_.as<cplx<T>>(), (const cplx<T>*)psi_.as<cplx<T>>(), N, M_,
                            corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(),
                            int(cap_), int(nyo_), int(nxo_), ntx_, T(p.obj_step));
+        });
       });
     }
     if (upd_probe) {
@@ -4535,8 +4586,8 @@ class Engine : public EngineBase {
                            dPm_.as<cplx<T>>(), tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_times_q<T, true>), dim3((n + 255) / 256, M_), dim3(256), 0,
                            stream_, dPm_.as<cplx<T>>(), (const cplx<T>*)q_.as<cplx<T>>(), n);
-        hipLaunchKernelGGL(k_probe_apply<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                           P_.as<cplx<T>>(), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
+        hipLaunchKernelGGL(k_probe_apply<T>, dim3(chunk_blocks(total, 1)), dim3(THREADS), 0,
+                           stream_, P_.as<cplx<T>>(), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
                            (const cplx<T>*)dPm_.as<cplx<T>>(), 1, n, total, T(p.probe_step));
       });
     }
@@ -4631,8 +4682,8 @@ class Engine : public EngineBase {
     // λ0 = 1.2e-7·k/n per pixel and mode (ptyrs/src/engine/lsqml.rs:31-33), summed over both.
     const double lam = 1.2e-7 * scale_ * double(M_);
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_probe_mean<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                         dPm_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, nb);
+      hipLaunchKernelGGL(k_probe_mean<T>, dim3(chunk_blocks(total, nchunk)), dim3(THREADS), 0,
+                         stream_, dPm_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, nb);
     });
     run(K_DOTS, [&] {
       // The direction as the slots read it: its sampled windows (the object's spectrum is no
@@ -4728,8 +4779,8 @@ class Engine : public EngineBase {
     if (upd_probe) {
       const int total = int(nprobe_ * n);
       run(K_PROBE, [&] {
-        hipLaunchKernelGGL(k_probe_apply<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                           P_.as<cplx<T>>(), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
+        hipLaunchKernelGGL(k_probe_apply<T>, dim3(chunk_blocks(total, nchunk)), dim3(THREADS), 0,
+                           stream_, P_.as<cplx<T>>(), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
                            dP_.as<cplx<T>>(), nchunk, n, total, T(p.probe_step / nb));
       });
     }

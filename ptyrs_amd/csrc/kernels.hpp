@@ -753,20 +753,65 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_rpie
   }
 }
 
-// P += s·Σ_chunks dP_part, then Wt = P·q (and, with W2, |Wt|²), at element i.
-template <typename T>
-__device__ __forceinline__ void probe_apply_at(int i, cplx<T>* __restrict__ P,
-                                               cplx<T>* __restrict__ Wt,
-                                               const cplx<T>* __restrict__ q,
-                                               const cplx<T>* __restrict__ dP_part, int nchunk,
-                                               int n, int total, T s, T* __restrict__ W2) {
-  if (i >= total) return;
-  kahan<T> sr, si;
-  for (int c = 0; c < nchunk; ++c) {
-    cplx<T> d = ld(dP_part + (size_t)c * total + i);
-    sr.add(d.x);
-    si.add(d.y);
+// Complex sums over `nchunk` planes of `total` values: a workgroup of BT threads takes PX
+// neighbouring elements, its BT/PX thread groups a contiguous share of the chunks each, and the
+// groups' Kahan pairs meet in LDS in group order. `part` holds 4·BT values. Returns true in the
+// threads (group 0) that hold the element's sum. With many chunks a thread walking all of them
+// is a chain of dependent-in-time loads (100 chunks at 64²: 28 µs of rPIE's update launch).
+template <typename T, int BT>
+__device__ __forceinline__ bool chunk_sum(const cplx<T>* __restrict__ src, int nchunk, int total,
+                                          int i, int px, T* part, kahan<T>& sr, kahan<T>& si) {
+  const int ng = BT / px, g = int(threadIdx.x) / px;
+  const int per = (nchunk + ng - 1) / ng;
+  const int c1 = (g + 1) * per < nchunk ? (g + 1) * per : nchunk;
+  if (i < total) {
+    constexpr int CU = 4;  // chunks loaded together, added in chunk order
+    for (int c0 = g * per; c0 < c1; c0 += CU) {
+      cplx<T> d[CU];
+#pragma unroll
+      for (int u = 0; u < CU; ++u)
+        if (c0 + u < c1) d[u] = ld(src + (size_t)(c0 + u) * total + i);
+#pragma unroll
+      for (int u = 0; u < CU; ++u)
+        if (c0 + u < c1) {
+          sr.add(d[u].x);
+          si.add(d[u].y);
+        }
+    }
   }
+  if (ng > 1) {
+    const int t = threadIdx.x;
+    part[t] = sr.s;
+    part[BT + t] = sr.c;
+    part[2 * BT + t] = si.s;
+    part[3 * BT + t] = si.c;
+    __syncthreads();
+    if (g == 0)
+      for (int k = 1; k < ng; ++k) {
+        sr.merge(part[k * px + t], part[BT + k * px + t]);
+        si.merge(part[2 * BT + k * px + t], part[3 * BT + k * px + t]);
+      }
+  }
+  return g == 0 && i < total;
+}
+
+// Elements per workgroup of BT threads for a sum over `nchunk` chunks: one thread per element
+// while a thread has few chunks to walk, else a wave of elements and BT/64 chunk groups.
+__host__ __device__ constexpr int chunk_px(int nchunk, int bt) { return nchunk < 16 ? bt : 64; }
+
+// P += s·Σ_chunks dP_part, then Wt = P·q (and, with W2, |Wt|²), for the elements of workgroup
+// `blk` (chunk_px of them).
+template <typename T, int BT>
+__device__ __forceinline__ void probe_apply_blk(int blk, cplx<T>* __restrict__ P,
+                                                cplx<T>* __restrict__ Wt,
+                                                const cplx<T>* __restrict__ q,
+                                                const cplx<T>* __restrict__ dP_part, int nchunk,
+                                                int n, int total, T s, T* __restrict__ W2,
+                                                T* part) {
+  const int px = chunk_px(nchunk, BT);
+  const int i = blk * px + int(threadIdx.x) % px;
+  kahan<T> sr, si;
+  if (!chunk_sum<T, BT>(dP_part, nchunk, total, i, px, part, sr, si)) return;
   cplx<T> p = ld(P + i);
   p = p + cplx<T>{sr.s, si.s} * s;
   st(P + i, p);
@@ -776,40 +821,88 @@ __device__ __forceinline__ void probe_apply_at(int i, cplx<T>* __restrict__ P,
 }
 
 template <typename T>
-__global__ void k_probe_apply(cplx<T>* __restrict__ P, cplx<T>* __restrict__ Wt,
-                              const cplx<T>* __restrict__ q, const cplx<T>* __restrict__ dP_part,
-                              int nchunk, int n, int total, T s) {
-  probe_apply_at(int(blockIdx.x * blockDim.x + threadIdx.x), P, Wt, q, dP_part, nchunk, n, total,
-                 s, (T*)nullptr);
+__global__ __launch_bounds__(THREADS) void k_probe_apply(
+    cplx<T>* __restrict__ P, cplx<T>* __restrict__ Wt, const cplx<T>* __restrict__ q,
+    const cplx<T>* __restrict__ dP_part, int nchunk, int n, int total, T s) {
+  __shared__ T part[4 * THREADS];
+  probe_apply_blk<T, THREADS>(int(blockIdx.x), P, Wt, q, dP_part, nchunk, n, total, s,
+                              (T*)nullptr, part);
 }
 
 // ---- object tiles --------------------------------------------------------------------------------
-// Object tiles of 64×4 pixels, one pixel per thread (TROWS rows per thread in general).
-constexpr int TILE_X = 64, TILE_Y = 4, TROWS = TILE_Y / (THREADS / TILE_X);
+// Object tiles of 64×4 pixels. A tile's workgroup has SP groups of THREADS threads, each with
+// one thread per pixel; a round stages up to THREADS of the tile's views in LDS, group g takes
+// the g-th contiguous share of them, and the groups' sums meet in LDS in group order. A pixel's
+// views are a serial chain of loads and compensated adds, so with few tiles the chip idles and
+// the chain is the time: SP = 4 below kSplitTiles tiles (tile_split), 1 above, where the tiles
+// alone fill it and the split would only add its combination. SP = 1 → 4, complex64: rPIE's
+// overlaps 22.8 → 10.8 µs and updates 31 → 11.4 (126 tiles, 64² frames, 100 views), LSQML's object
+// direction 89 → 25 µs (400 tiles, 128 views of 128² × 2 modes); at 5076 tiles SP = 1 runs.
+constexpr int TILE_X = 64, TILE_Y = 4;
+static_assert(TILE_X * TILE_Y == THREADS, "a tile has one thread per pixel");
+constexpr int kSplitTiles = 2048;
+
+// Views [lo, hi) of a round of k staged views that group g of SP takes.
+template <int SP>
+__device__ __forceinline__ int2 share_of(int g, int k) {
+  if constexpr (SP == 1) return int2{0, k};
+  const int per = (k + SP - 1) / SP;
+  const int lo = g * per, hi = lo + per;
+  return int2{lo < k ? lo : k, hi < k ? hi : k};
+}
+
+// The groups' complex Kahan sums into group 0's, in group order. `part` holds
+// 4·(SP − 1)·THREADS values; all threads call it.
+template <typename T, int SP>
+__device__ __forceinline__ void merge_groups(kahan<T>& sr, kahan<T>& si, T* part, int g, int p) {
+  if constexpr (SP > 1) {
+    constexpr int W = (SP - 1) * THREADS;
+    if (g > 0) {
+      T* d = part + (g - 1) * THREADS + p;
+      d[0] = sr.s;
+      d[W] = sr.c;
+      d[2 * W] = si.s;
+      d[3 * W] = si.c;
+    }
+    __syncthreads();
+    if (g == 0) {
+#pragma unroll
+      for (int k = 0; k < SP - 1; ++k) {
+        const T* d = part + k * THREADS + p;
+        sr.merge(d[0], d[W]);
+        si.merge(d[2 * W], d[3 * W]);
+      }
+    }
+  }
+}
 
 // One workgroup per object tile: (1) the batch slots whose N×N window meets the tile, in slot
 // order, compacted with wave ballots into list[tile][·] and count[tile]; (2) with `W2` (|W_m|²
 // per mode, W = P·q) or `Wv` (every view's own wave W, plane slot·M + m, under position
 // offsets), each pixel's batch overlap D_m = Σ_views |W_m|² per mode into D[m][pixel] and the
 // tile max of Σ_m D_m (rPIE's regulariser max).
-template <typename T>
-__global__ __launch_bounds__(THREADS) void k_bin_tiles(
+template <typename T, int SP>
+__global__ __launch_bounds__(THREADS * SP) void k_bin_tiles(
     const int2* __restrict__ corner, const int* __restrict__ order, int nb, int N, int ntx,
     int cap, int* __restrict__ list, int* __restrict__ count, const T* __restrict__ W2,
     int M, int nyo, int nxo, T* __restrict__ D, T* __restrict__ tilemax,
     const cplx<T>* __restrict__ Wv) {
-  __shared__ int wave_n[THREADS / 64];
+  constexpr int BT = THREADS * SP;
+  constexpr int MM = 4;  // modes per chunk of overlaps held in registers
+  __shared__ int wave_n[BT / 64];
   __shared__ int base_s;
-  __shared__ T red[THREADS];
+  __shared__ T red[BT];
+  __shared__ T part[SP > 1 ? (SP - 1) * MM * THREADS : 1];
   // The corners (and batch slots) of the tile's first THREADS views, kept as they are found.
   __shared__ int2 cs[THREADS];
   __shared__ int bs[THREADS];
   const int t = tile_id(), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int g = tid / THREADS, px = tid % THREADS;
   const int ty0 = (t / ntx) * TILE_Y, tx0 = (t % ntx) * TILE_X;
   int* out = list + (size_t)t * cap;
   if (tid == 0) base_s = 0;
   __syncthreads();
-  for (int s = 0; s < nb; s += THREADS) {
+  for (int s = 0; s < nb; s += BT) {
     const int b = s + tid;
     bool hit = false;
     int2 c = {0, 0};
@@ -833,7 +926,7 @@ __global__ __launch_bounds__(THREADS) void k_bin_tiles(
     __syncthreads();
     if (tid == 0) {
       int tot = 0;
-      for (int w = 0; w < THREADS / 64; ++w) tot += wave_n[w];
+      for (int w = 0; w < BT / 64; ++w) tot += wave_n[w];
       base_s += tot;
     }
     __syncthreads();
@@ -842,83 +935,74 @@ __global__ __launch_bounds__(THREADS) void k_bin_tiles(
   if (tid == 0) count[t] = nl;
   if (W2 == nullptr && Wv == nullptr) return;
   // Modes in chunks of MM, each chunk's overlaps in registers; Σ_m D_m in mode order.
-  constexpr int MM = 4;
-  const int X = tx0 + tid % TILE_X, Y0 = ty0 + tid / TILE_X;
-  constexpr int RS = THREADS / TILE_X;  // row stride between a thread's pixels
+  const int X = tx0 + px % TILE_X, Y = ty0 + px / TILE_X;
   const int n = N * N;
   const size_t no = (size_t)nyo * nxo;
-  T tot[TROWS] = {};
+  T tot = 0;
   for (int m0 = 0; m0 < M; m0 += MM) {
-  const int mc = M - m0 < MM ? M - m0 : MM;
-  T dm[TROWS][MM] = {};
-  for (int s = 0; s < nl; s += THREADS) {
-    const int k = nl - s < THREADS ? nl - s : THREADS;
-    if (s > 0 || (m0 > 0 && nl > THREADS)) {
-      if (tid < k) {
-        bs[tid] = out[s + tid];
-        cs[tid] = corner[order[bs[tid]]];
+    const int mc = M - m0 < MM ? M - m0 : MM;
+    T dm[MM] = {};
+    for (int s = 0; s < nl; s += THREADS) {
+      const int k = nl - s < THREADS ? nl - s : THREADS;
+      if (s > 0 || (m0 > 0 && nl > THREADS)) {
+        if (tid < k) {
+          bs[tid] = out[s + tid];
+          cs[tid] = corner[order[bs[tid]]];
+        }
+        __syncthreads();
+      }
+      if (X < nxo) {
+        // One slot at a time in this form is fastest (256² × 4 modes: 2 slots' loads together
+        // took 8 % longer, 4 slots 14 %, 8 slots 30 %, and a plain loop with the bounds test
+        // as a branch 31 %).
+        const int2 r = share_of<SP>(g, k);
+        for (int i = r.x; i < r.y; ++i) {
+          const int x = X - cs[i].y, y = Y - cs[i].x;
+          const bool ok = x >= 0 && x < N && y >= 0 && y < N;
+          T w2[MM];
+          if (ok) {
+#pragma unroll
+            for (int m = 0; m < MM; ++m)
+              if (m < mc)
+                w2[m] = Wv ? norm2(Wv[((size_t)bs[i] * M + m0 + m) * n + y * N + x])
+                           : W2[(size_t)(m0 + m) * n + y * N + x];
+          }
+          if (ok) {
+#pragma unroll
+            for (int m = 0; m < MM; ++m)
+              if (m < mc) dm[m] += w2[m];
+          }
+        }
       }
       __syncthreads();
     }
-    if (X < nxo) {
-      // SU slots per step, added in slot order. One slot at a time in this form is fastest
-      // (256² × 4 modes: 2 slots took 8 % longer, 4 slots 14 %, 8 slots 30 %, and a plain
-      // loop with the bounds test as a branch 31 %).
-      constexpr int SU = 1;
-      for (int i0 = 0; i0 < k; i0 += SU) {
+    if constexpr (SP > 1) {
+      if (g > 0) {
 #pragma unroll
-        for (int r = 0; r < TROWS; ++r) {
-          T w2[SU][MM];
-          bool ok[SU];
-#pragma unroll
-          for (int u = 0; u < SU; ++u) {
-            const int i = i0 + u < k ? i0 + u : k - 1;  // cs holds k entries
-            const int x = X - cs[i].y, y = Y0 + RS * r - cs[i].x;
-            ok[u] = i0 + u < k && x >= 0 && x < N && y >= 0 && y < N;
-            if (ok[u]) {
-#pragma unroll
-              for (int m = 0; m < MM; ++m)
-                if (m < mc)
-                  w2[u][m] = Wv ? norm2(Wv[((size_t)bs[i] * M + m0 + m) * n + y * N + x])
-                                : W2[(size_t)(m0 + m) * n + y * N + x];
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < SU; ++u)
-            if (ok[u]) {
-#pragma unroll
-              for (int m = 0; m < MM; ++m)
-                if (m < mc) dm[r][m] += w2[u][m];
-            }
-        }
+        for (int m = 0; m < MM; ++m) part[((g - 1) * MM + m) * THREADS + px] = dm[m];
       }
-    }
-    __syncthreads();
-  }
-  if (X < nxo && nl > 0) {
+      __syncthreads();
+      if (g == 0) {
 #pragma unroll
-    for (int r = 0; r < TROWS; ++r) {
-      const int Y = Y0 + RS * r;
-      if (Y >= nyo) continue;
+        for (int k = 0; k < SP - 1; ++k)
+#pragma unroll
+          for (int m = 0; m < MM; ++m) dm[m] += part[(k * MM + m) * THREADS + px];
+      }
+      __syncthreads();
+    }
+    if (g == 0 && X < nxo && nl > 0 && Y < nyo) {
       const size_t p = (size_t)Y * nxo + X;
       T s = 0;
 #pragma unroll
       for (int m = 0; m < MM; ++m)
         if (m < mc) {
-          D[(m0 + m) * no + p] = dm[r][m];
-          s += dm[r][m];
+          D[(m0 + m) * no + p] = dm[m];
+          s += dm[m];
         }
-      tot[r] += s;
+      tot += s;
     }
   }
-  }
-  T sum = 0;
-  if (X < nxo && nl > 0) {
-#pragma unroll
-    for (int r = 0; r < TROWS; ++r)
-      if (Y0 + RS * r < nyo) sum = tot[r] > sum ? tot[r] : sum;
-  }
-  T r = block_reduce<THREADS>(sum, red, MaxOp());
+  T r = block_reduce<BT>(tot, red, MaxOp());
   if (tid == 0) tilemax[t] = r;
 }
 
@@ -938,20 +1022,20 @@ __global__ __launch_bounds__(MAX_THREADS) void k_max_reduce(const T* __restrict_
 // plane, every mode's term already divided by its denominator): every object pixel owned by one
 // thread adds, in slot order and Kahan-compensated, the terms of the views over it, then
 // O += step·Σ. No atomics; the result does not depend on the launch shape.
-template <typename T>
+template <typename T, int SP>
 __device__ __forceinline__ void obj_update_rpie_tile(
     int t, cplx<T>* __restrict__ O, const cplx<T>* __restrict__ wsum, int N, int M,
     const int2* __restrict__ corner, const int* __restrict__ order, const int* __restrict__ list,
-    const int* __restrict__ count, int cap, int nyo, int nxo, int ntx, T step) {
-  constexpr int RS = THREADS / TILE_X;
+    const int* __restrict__ count, int cap, int nyo, int nxo, int ntx, T step, T* part) {
   __shared__ int3 cs[THREADS];
-  const int tid = threadIdx.x;
-  const int X = (t % ntx) * TILE_X + tid % TILE_X, Y0 = (t / ntx) * TILE_Y + tid / TILE_X;
+  __shared__ unsigned char hit[SP > 1 ? (SP - 1) * THREADS : 1];
+  const int tid = threadIdx.x, g = tid / THREADS, px = tid % THREADS;
+  const int X = (t % ntx) * TILE_X + px % TILE_X, Y = (t / ntx) * TILE_Y + px / TILE_X;
   const int nl = count[t];
   if (nl == 0) return;
   const int n = N * N;
-  kahan<T> nr[TROWS], ni[TROWS];
-  bool covered[TROWS] = {};
+  kahan<T> nr, ni;
+  bool covered = false;
   const int* lst = list + (size_t)t * cap;
   for (int s = 0; s < nl; s += THREADS) {
     const int k = nl - s < THREADS ? nl - s : THREADS;
@@ -963,63 +1047,67 @@ __device__ __forceinline__ void obj_update_rpie_tile(
     __syncthreads();
     // SU slots per step: their loads are issued together, then added in slot order.
     constexpr int SU = 4;
-    for (int i0 = 0; i0 < k && X < nxo; i0 += SU) {
+    const int2 sh = share_of<SP>(g, k);
+    for (int i0 = sh.x; i0 < sh.y && X < nxo; i0 += SU) {
+      cplx<T> v[SU];
+      bool ok[SU];
 #pragma unroll
-      for (int r = 0; r < TROWS; ++r) {
-        cplx<T> g[SU];
-        bool ok[SU];
-#pragma unroll
-        for (int u = 0; u < SU; ++u) {
-          const int i = i0 + u < k ? i0 + u : k - 1;  // cs holds k entries
-          const int x = X - cs[i].z, y = Y0 + RS * r - cs[i].y;
-          ok[u] = i0 + u < k && x >= 0 && x < N && y >= 0 && y < N;
-          if (ok[u]) g[u] = ld(wsum + (size_t)cs[i].x * M * n + y * N + x);
-        }
-#pragma unroll
-        for (int u = 0; u < SU; ++u)
-          if (ok[u]) {
-            nr[r].add(g[u].x);
-            ni[r].add(g[u].y);
-            covered[r] = true;
-          }
+      for (int u = 0; u < SU; ++u) {
+        const int i = i0 + u < sh.y ? i0 + u : sh.y - 1;
+        const int x = X - cs[i].z, y = Y - cs[i].y;
+        ok[u] = i0 + u < sh.y && x >= 0 && x < N && y >= 0 && y < N;
+        if (ok[u]) v[u] = ld(wsum + (size_t)cs[i].x * M * n + y * N + x);
       }
+#pragma unroll
+      for (int u = 0; u < SU; ++u)
+        if (ok[u]) {
+          nr.add(v[u].x);
+          ni.add(v[u].y);
+          covered = true;
+        }
     }
     __syncthreads();
   }
+  if constexpr (SP > 1) {
+    if (g > 0) hit[(g - 1) * THREADS + px] = covered;
+    merge_groups<T, SP>(nr, ni, part, g, px);
+    if (g > 0) return;
 #pragma unroll
-  for (int r = 0; r < TROWS; ++r) {
-    const int Y = Y0 + RS * r;
-    if (!covered[r] || Y >= nyo) continue;
-    cplx<T>* o = O + (size_t)Y * nxo + X;
-    st(o, ld(o) + cplx<T>{nr[r].s, ni[r].s} * step);
+    for (int k = 0; k < SP - 1; ++k) covered |= hit[k * THREADS + px] != 0;
   }
+  if (!covered || Y >= nyo) return;
+  cplx<T>* o = O + (size_t)Y * nxo + X;
+  st(o, ld(o) + cplx<T>{nr.s, ni.s} * step);
 }
 
-template <typename T>
-__global__ __launch_bounds__(THREADS) void k_obj_update_rpie_sum(
+template <typename T, int SP>
+__global__ __launch_bounds__(THREADS * SP) void k_obj_update_rpie_sum(
     cplx<T>* __restrict__ O, const cplx<T>* __restrict__ wsum, int N, int M,
     const int2* __restrict__ corner, const int* __restrict__ order, const int* __restrict__ list,
     const int* __restrict__ count, int cap, int nyo, int nxo, int ntx, T step) {
-  obj_update_rpie_tile(tile_id(), O, wsum, N, M, corner, order, list, count, cap, nyo, nxo, ntx,
-                       step);
+  __shared__ T part[SP > 1 ? 4 * (SP - 1) * THREADS : 1];
+  obj_update_rpie_tile<T, SP>(tile_id(), O, wsum, N, M, corner, order, list, count, cap, nyo,
+                              nxo, ntx, step, part);
 }
 
-// The object update's ntile workgroups and then the probe update's (THREADS elements each) in
+// The object update's ntile workgroups and then the probe update's (chunk_px elements each) in
 // one launch: the two read and write disjoint buffers. The probe update also leaves |W_m|² of
 // the new probe terms in W2 for the next batch's overlaps.
-template <typename T>
-__global__ __launch_bounds__(THREADS) void k_rpie_updates(
+template <typename T, int SP>
+__global__ __launch_bounds__(THREADS * SP) void k_rpie_updates(
     cplx<T>* __restrict__ O, const cplx<T>* __restrict__ wsum, int N, int M,
     const int2* __restrict__ corner, const int* __restrict__ order, const int* __restrict__ list,
     const int* __restrict__ count, int cap, int nyo, int nxo, int ntx, T step, int ntile,
     cplx<T>* __restrict__ P, cplx<T>* __restrict__ Wt, const cplx<T>* __restrict__ q,
     const cplx<T>* __restrict__ dP_part, int nchunk, int total, T pstep, T* __restrict__ W2) {
+  constexpr int BT = THREADS * SP;
+  __shared__ T part[4 * BT];
   if (int(blockIdx.x) < ntile)
-    obj_update_rpie_tile(int(blockIdx.x), O, wsum, N, M, corner, order, list, count, cap, nyo,
-                         nxo, ntx, step);
+    obj_update_rpie_tile<T, SP>(int(blockIdx.x), O, wsum, N, M, corner, order, list, count, cap,
+                                nyo, nxo, ntx, step, part);
   else
-    probe_apply_at(int((blockIdx.x - ntile) * THREADS + threadIdx.x), P, Wt, q, dP_part, nchunk,
-                   N * N, total, pstep, W2);
+    probe_apply_blk<T, BT>(int(blockIdx.x) - ntile, P, Wt, q, dP_part, nchunk, N * N, total,
+                           pstep, W2, part);
 }
 
 // ---- LSQML ------------------------------------------------------------------------------------------
@@ -1093,20 +1181,20 @@ __global__ __launch_bounds__(THREADS) void k_lsqml_xi_sums(
 // ([slot][n]) with q_frame. With `accumulate` the result is added to dO.
 // ptyrs/src/engine/lsqml.rs:183-188, :587-598; ptyrs/src/engine/ops.rs:279-310;
 // ptyrs/src/engine/multislice.rs:402-430
-template <typename T>
-__global__ __launch_bounds__(THREADS) void k_lsqml_obj_dir(
+template <typename T, int SP, int MM>
+__global__ __launch_bounds__(THREADS * SP) void k_lsqml_obj_dir(
     cplx<T>* __restrict__ dO, const cplx<T>* __restrict__ Wt, const cplx<T>* __restrict__ chi,
     int N, int M, const int2* __restrict__ corner, const int* __restrict__ order,
     const int* __restrict__ list, const int* __restrict__ count, int cap, int nyo, int nxo,
-    int ntx, const T* __restrict__ pre, const T* __restrict__ floor, int per_view = 0,
-    const cplx<T>* __restrict__ q = nullptr, int q_frame = 0, int accumulate = 0) {
-  constexpr int RS = THREADS / TILE_X;
+    int ntx, const T* __restrict__ pre, const T* __restrict__ floor, int per_view,
+    const cplx<T>* __restrict__ q, int q_frame, int accumulate) {
   __shared__ int3 cs[THREADS];
-  const int t = tile_id(), tid = threadIdx.x;
-  const int X = (t % ntx) * TILE_X + tid % TILE_X, Y0 = (t / ntx) * TILE_Y + tid / TILE_X;
+  __shared__ T part[SP > 1 ? 4 * (SP - 1) * THREADS : 1];
+  const int t = tile_id(), tid = threadIdx.x, g = tid / THREADS, px = tid % THREADS;
+  const int X = (t % ntx) * TILE_X + px % TILE_X, Y = (t / ntx) * TILE_Y + px / TILE_X;
   const int nl = count[t];
   const int n = N * N;
-  kahan<T> sr[TROWS], si[TROWS];
+  kahan<T> sr, si;
   const int* lst = list + (size_t)t * cap;
   for (int s = 0; s < nl; s += THREADS) {
     const int k = nl - s < THREADS ? nl - s : THREADS;
@@ -1116,59 +1204,71 @@ __global__ __launch_bounds__(THREADS) void k_lsqml_obj_dir(
       cs[tid] = int3{b, c.x, c.y};
     }
     __syncthreads();
-    for (int i = 0; i < k && X < nxo; ++i) {
-      const int x = X - cs[i].z;
-      if (x < 0 || x >= N) continue;
-      const cplx<T>* cv = chi + (size_t)cs[i].x * M * n;
-      const cplx<T>* wv = per_view ? Wt + (size_t)cs[i].x * M * n : Wt;
-      const cplx<T>* qv = q && q_frame ? q + (size_t)cs[i].x * n : q;
+    // SU slots of MM modes per step: their loads are issued together, then added in slot order.
+    constexpr int SU = 4 / MM;
+    const int2 sh = share_of<SP>(g, k);
+    for (int i0 = sh.x; i0 < sh.y && X < nxo; i0 += SU) {
+      int j[SU];
+      size_t cv[SU];
+      bool ok[SU];
+      cplx<T> qj[SU];
 #pragma unroll
-      for (int r = 0; r < TROWS; ++r) {
-        const int y = Y0 + RS * r - cs[i].y;
-        if (y < 0 || y >= N) continue;
-        const int j = y * N + x;
-        for (int m = 0; m < M; ++m) {
-          cplx<T> w = ld(wv + (size_t)m * n + j);
-          if (qv) w = w * ld(qv + j);
-          const cplx<T> g = cmulc(w, ld(cv + (size_t)m * n + j));
-          sr[r].add(g.x);
-          si[r].add(g.y);
-        }
+      for (int u = 0; u < SU; ++u) {
+        const int i = i0 + u < sh.y ? i0 + u : sh.y - 1;
+        const int x = X - cs[i].z, y = Y - cs[i].y;
+        ok[u] = i0 + u < sh.y && x >= 0 && x < N && y >= 0 && y < N;
+        j[u] = y * N + x;
+        cv[u] = (size_t)cs[i].x * M * n;
+        if (q && ok[u]) qj[u] = ld(q + (q_frame ? (size_t)cs[i].x * n : 0) + j[u]);
+      }
+      for (int m0 = 0; m0 < M; m0 += MM) {
+        cplx<T> w[SU][MM], c[SU][MM];
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+#pragma unroll
+          for (int m = 0; m < MM; ++m)
+            if (ok[u] && m0 + m < M) {
+              const size_t p = (size_t)(m0 + m) * n + j[u];
+              w[u][m] = ld(Wt + (per_view ? cv[u] : 0) + p);
+              c[u][m] = ld(chi + cv[u] + p);
+            }
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+#pragma unroll
+          for (int m = 0; m < MM; ++m)
+            if (ok[u] && m0 + m < M) {
+              const cplx<T> v = cmulc(q ? w[u][m] * qj[u] : w[u][m], c[u][m]);
+              sr.add(v.x);
+              si.add(v.y);
+            }
       }
     }
     __syncthreads();
   }
-  if (X >= nxo) return;
-  const T fl = pre ? floor[0] : T(0);
-#pragma unroll
-  for (int r = 0; r < TROWS; ++r) {
-    const int Y = Y0 + RS * r;
-    if (Y >= nyo) continue;
-    const size_t p = (size_t)Y * nxo + X;
-    T inv = T(1);
-    if (pre) {
-      const T pr = pre[p];
-      inv = T(1) / sqrt(pr * pr + fl);
-    }
-    cplx<T> v = cplx<T>{sr[r].s * inv, si[r].s * inv};
-    if (accumulate) v = v + ld(dO + p);
-    st(dO + p, v);
+  merge_groups<T, SP>(sr, si, part, g, px);
+  if (g > 0 || X >= nxo || Y >= nyo) return;
+  const size_t p = (size_t)Y * nxo + X;
+  T inv = T(1);
+  if (pre) {
+    const T pr = pre[p];
+    inv = T(1) / sqrt(pr * pr + floor[0]);
   }
+  cplx<T> v = cplx<T>{sr.s * inv, si.s * inv};
+  if (accumulate) v = v + ld(dO + p);
+  st(dO + p, v);
 }
 
 // dP = Σ_chunks partials / nb (the frame mean of the probe directions).
 template <typename T>
-__global__ void k_probe_mean(cplx<T>* __restrict__ dP, const cplx<T>* __restrict__ dP_part,
-                             int nchunk, int total, int nb) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
+__global__ __launch_bounds__(THREADS) void k_probe_mean(cplx<T>* __restrict__ dP,
+                                                        const cplx<T>* __restrict__ dP_part,
+                                                        int nchunk, int total, int nb) {
+  __shared__ T part[4 * THREADS];
+  const int px = chunk_px(nchunk, THREADS);
+  const int i = int(blockIdx.x) * px + int(threadIdx.x) % px;
   kahan<T> sr, si;
-  for (int c = 0; c < nchunk; ++c) {
-    cplx<T> d = ld(dP_part + (size_t)c * total + i);
-    sr.add(d.x);
-    si.add(d.y);
-  }
-  st(dP + i, cplx<T>{sr.s, si.s} * (T(1) / T(nb)));
+  if (chunk_sum<T, THREADS>(dP_part, nchunk, total, i, px, part, sr, si))
+    st(dP + i, cplx<T>{sr.s, si.s} * (T(1) / T(nb)));
 }
 
 // Per slot and workgroup the six sums of the step-size system (FP64):
@@ -1297,48 +1397,49 @@ __global__ void k_lsqml_apply_probe(cplx<T>* __restrict__ P, cplx<T>* __restrict
 
 // Illumination Σ_m Σ_views |P_m|² over a tile list's views, added into illum (each pixel owned
 // by one thread).
-template <typename T>
-__global__ __launch_bounds__(THREADS) void k_illumination(
+template <typename T, int SP>
+__global__ __launch_bounds__(THREADS * SP) void k_illumination(
     T* __restrict__ illum, const cplx<T>* __restrict__ P, int N, int M,
     const int2* __restrict__ corner, const int* __restrict__ order, const int* __restrict__ list,
     const int* __restrict__ count, int cap, int nyo, int nxo, int ntx) {
-  constexpr int RS = THREADS / TILE_X;
   __shared__ int2 cs[THREADS];
-  const int t = tile_id(), tid = threadIdx.x;
-  const int X = (t % ntx) * TILE_X + tid % TILE_X, Y0 = (t / ntx) * TILE_Y + tid / TILE_X;
+  __shared__ T part[SP > 1 ? (SP - 1) * THREADS : 1];
+  const int t = tile_id(), tid = threadIdx.x, g = tid / THREADS, px = tid % THREADS;
+  const int X = (t % ntx) * TILE_X + px % TILE_X, Y = (t / ntx) * TILE_Y + px / TILE_X;
   const int nl = count[t];
   const int n = N * N;
-  T sum[TROWS] = {};
+  T sum = 0;
   for (int s = 0; s < nl; s += THREADS) {
     const int k = nl - s < THREADS ? nl - s : THREADS;
     if (tid < k) cs[tid] = corner[order[list[(size_t)t * cap + s + tid]]];
     __syncthreads();
     // SU views per step: their loads issued together, added in view order.
     constexpr int SU = 8;
-    for (int i0 = 0; i0 < k && X < nxo; i0 += SU) {
+    const int2 sh = share_of<SP>(g, k);
+    for (int i0 = sh.x; i0 < sh.y && X < nxo; i0 += SU) {
+      T a[SU];
 #pragma unroll
-      for (int r = 0; r < TROWS; ++r) {
-        T a[SU];
-#pragma unroll
-        for (int u = 0; u < SU; ++u) {
-          const int i = i0 + u < k ? i0 + u : k - 1;  // cs holds k entries
-          const int x = X - cs[i].y, y = Y0 + RS * r - cs[i].x;
-          a[u] = 0;
-          if (i0 + u < k && x >= 0 && x < N && y >= 0 && y < N)
-            for (int m = 0; m < M; ++m) a[u] += norm2(ld(P + (size_t)m * n + y * N + x));
-        }
-#pragma unroll
-        for (int u = 0; u < SU; ++u) sum[r] += a[u];
+      for (int u = 0; u < SU; ++u) {
+        const int i = i0 + u < sh.y ? i0 + u : sh.y - 1;
+        const int x = X - cs[i].y, y = Y - cs[i].x;
+        a[u] = 0;
+        if (i0 + u < sh.y && x >= 0 && x < N && y >= 0 && y < N)
+          for (int m = 0; m < M; ++m) a[u] += norm2(ld(P + (size_t)m * n + y * N + x));
       }
+#pragma unroll
+      for (int u = 0; u < SU; ++u) sum += a[u];
     }
     __syncthreads();
   }
-  if (X >= nxo || nl == 0) return;
+  if constexpr (SP > 1) {
+    if (g > 0) part[(g - 1) * THREADS + px] = sum;
+    __syncthreads();
+    if (g > 0) return;
 #pragma unroll
-  for (int r = 0; r < TROWS; ++r) {
-    const int Y = Y0 + RS * r;
-    if (Y < nyo) illum[(size_t)Y * nxo + X] += sum[r];
+    for (int k = 0; k < SP - 1; ++k) sum += part[k * THREADS + px];
   }
+  if (X >= nxo || nl == 0) return;
+  if (Y < nyo) illum[(size_t)Y * nxo + X] += sum;
 }
 
 // pre = (pre + illum)/2, or on the first update (illum·init + illum)/2; pre's max goes to
@@ -2111,31 +2212,44 @@ __global__ __launch_bounds__(THREADS) void k_probe_sums(
 }
 
 // Sums the probe partials over chunks (Kahan) into num[M][n] and den[n], and writes the per
-// workgroup max of den for the regulariser.
+// workgroup max of den for the regulariser. Grid (ceil(n/64), M + 1) of REDUCE_THREADS: 64
+// pixels of one mode's num (or, y = M, of den), the chunks shared out over 16 thread groups.
+// One thread per pixel walking every chunk of every mode left 3/4 of the CUs idle at 128² and
+// took 252 µs for 256 chunks of 2 modes; this takes 21.
+constexpr int REDUCE_THREADS = 1024, REDUCE_PX = 64;
 template <typename T>
-__global__ __launch_bounds__(THREADS) void k_probe_reduce(
+__global__ __launch_bounds__(REDUCE_THREADS) void k_probe_reduce(
     const cplx<T>* __restrict__ num_part, const T* __restrict__ den_part, int nchunk, int n, int M,
     cplx<T>* __restrict__ num, T* __restrict__ den, T* __restrict__ maxpart) {
-  __shared__ T red[THREADS];
-  const int i = blockIdx.x * THREADS + threadIdx.x;
+  constexpr int BT = REDUCE_THREADS, NG = BT / REDUCE_PX;
+  __shared__ T part[4 * BT];
+  const int tid = threadIdx.x, p = tid % REDUCE_PX, g = tid / REDUCE_PX, m = blockIdx.y;
+  const int i = blockIdx.x * REDUCE_PX + p;
+  if (m < M) {
+    const int e = m * n + i;  // the element of a chunk's [M][n] planes; past n it is not summed
+    kahan<T> sr, si;
+    if (chunk_sum<T, BT>(num_part, nchunk, M * n, i < n ? e : M * n, REDUCE_PX, part, sr, si))
+      st(num + e, cplx<T>{sr.s, si.s});
+    return;
+  }
+  const int per = (nchunk + NG - 1) / NG;
+  const int c1 = (g + 1) * per < nchunk ? (g + 1) * per : nchunk;
+  kahan<T> d;
+  if (i < n)
+    for (int c = g * per; c < c1; ++c) d.add(den_part[(size_t)c * n + i]);
+  part[tid] = d.s;
+  part[BT + tid] = d.c;
+  __syncthreads();
+  if (g > 0) return;
+  for (int k = 1; k < NG; ++k) d.merge(part[k * REDUCE_PX + p], part[BT + k * REDUCE_PX + p]);
   T mx = 0;
   if (i < n) {
-    kahan<T> d;
-    for (int c = 0; c < nchunk; ++c) d.add(den_part[(size_t)c * n + i]);
     den[i] = d.s;
     mx = d.s;
-    for (int m = 0; m < M; ++m) {
-      kahan<T> sr, si;
-      for (int c = 0; c < nchunk; ++c) {
-        const cplx<T> v = ld(num_part + ((size_t)c * M + m) * n + i);
-        sr.add(v.x);
-        si.add(v.y);
-      }
-      st(num + (size_t)m * n + i, cplx<T>{sr.s, si.s});
-    }
   }
-  T r = block_reduce<THREADS>(mx, red, MaxOp());
-  if (threadIdx.x == 0) maxpart[blockIdx.x] = r;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = MaxOp()(mx, __shfl_xor(mx, off, 64));
+  if (p == 0) maxpart[blockIdx.x] = mx;
 }
 
 // PyNX blend of the probe: P = (num + reg·P)/max(den + reg, 1e-12), reg = inertia·max(den);
@@ -2158,15 +2272,16 @@ __global__ void k_probe_blend(cplx<T>* __restrict__ P, cplx<T>* __restrict__ Wt,
 // sums Σ_m Σ_views conj(W_m)·ψ_m (Kahan) in view order, and O = (num + reg·O)/max(norm + reg,
 // 1e-12) with norm = Σ_m D_m from k_bin_tiles and reg = inertia·max(norm). With w_view W is the
 // frame's own wave (plane frame·M + m of Wt, a moved probe; the order is every frame's).
-template <typename T, bool H = false>
-__global__ __launch_bounds__(THREADS) void k_obj_blend(
+template <typename T, bool H, int SP, int MM>
+__global__ __launch_bounds__(THREADS * SP) void k_obj_blend(
     cplx<T>* __restrict__ O, const cplx<T>* __restrict__ Wt, const T* __restrict__ D,
     Carried<T, H> carried, int N, int M, const int2* __restrict__ corner,
     const int* __restrict__ order, const int* __restrict__ list, const int* __restrict__ count,
-    int cap, int nyo, int nxo, int ntx, const T* __restrict__ nmax, T inertia, int w_view = 0) {
+    int cap, int nyo, int nxo, int ntx, const T* __restrict__ nmax, T inertia, int w_view) {
   __shared__ int3 cs[THREADS];
-  const int t = tile_id(), tid = threadIdx.x;
-  const int X = (t % ntx) * TILE_X + tid % TILE_X, Y = (t / ntx) * TILE_Y + tid / TILE_X;
+  __shared__ T part[SP > 1 ? 4 * (SP - 1) * THREADS : 1];
+  const int t = tile_id(), tid = threadIdx.x, g = tid / THREADS, px = tid % THREADS;
+  const int X = (t % ntx) * TILE_X + px % TILE_X, Y = (t / ntx) * TILE_Y + px / TILE_X;
   const int nl = count[t];
   const bool inside = X < nxo && Y < nyo;
   const int n = N * N;
@@ -2180,22 +2295,47 @@ __global__ __launch_bounds__(THREADS) void k_obj_blend(
       cs[tid] = int3{f, c.x, c.y};
     }
     __syncthreads();
-    for (int i = 0; i < k && inside; ++i) {
-      const int y = Y - cs[i].y, x = X - cs[i].z;
-      if (y >= 0 && y < N && x >= 0 && x < N) {
-        const int j = y * N + x;
-        const size_t cv = (size_t)cs[i].x * M * n + j;
-        const cplx<T>* wv = w_view ? Wt + (size_t)cs[i].x * M * n : Wt;
-        for (int m = 0; m < M; ++m) {
-          const cplx<T> g = cmulc(ld(wv + (size_t)m * n + j), carried.get(cv + (size_t)m * n));
-          sr.add(g.x);
-          si.add(g.y);
-        }
+    // SU views of MM modes per step: their loads are issued together, then added in view order.
+    constexpr int SU = 4 / MM;
+    const int2 sh = share_of<SP>(g, k);
+    for (int i0 = sh.x; i0 < sh.y && inside; i0 += SU) {
+      int j[SU];
+      size_t cv[SU];
+      bool ok[SU];
+#pragma unroll
+      for (int u = 0; u < SU; ++u) {
+        const int i = i0 + u < sh.y ? i0 + u : sh.y - 1;
+        const int y = Y - cs[i].y, x = X - cs[i].z;
+        ok[u] = i0 + u < sh.y && y >= 0 && y < N && x >= 0 && x < N;
+        j[u] = y * N + x;
+        cv[u] = (size_t)cs[i].x * M * n;
+      }
+      for (int m0 = 0; m0 < M; m0 += MM) {
+        cplx<T> w[SU][MM], c[SU][MM];
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+#pragma unroll
+          for (int m = 0; m < MM; ++m)
+            if (ok[u] && m0 + m < M) {
+              const size_t p = (size_t)(m0 + m) * n + j[u];
+              w[u][m] = ld(Wt + (w_view ? cv[u] : 0) + p);
+              c[u][m] = carried.get(cv[u] + p);
+            }
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+#pragma unroll
+          for (int m = 0; m < MM; ++m)
+            if (ok[u] && m0 + m < M) {
+              const cplx<T> v = cmulc(w[u][m], c[u][m]);
+              sr.add(v.x);
+              si.add(v.y);
+            }
       }
     }
     __syncthreads();
   }
-  if (!inside) return;
+  merge_groups<T, SP>(sr, si, part, g, px);
+  if (g > 0 || !inside) return;
   const size_t no = (size_t)nyo * nxo, p = (size_t)Y * nxo + X;
   T norm = 0;
   if (nl > 0)
