@@ -2359,11 +2359,22 @@ class Engine : public EngineBase {
   template <int LOAD, int STORE>
   void axis_pass(int axis, bool inverse, const cplx<T>* in, void* out, const AxisGeom& g,
                  int nplanes, PhaseArgs ph = PhaseArgs{nullptr, 0, 0, 0, 0}, T scale = T(1)) {
-    const AxisPlan& pl = fo_plan_[axis];
+    AxisPlan pl = fo_plan_[axis];
     const int L = pl.L;
-    const int G = std::max(1, std::min(16, 1024 / L));
+    const int odd = pl.nst ? pl.radix[pl.nst - 1] : 1;  // the plan's largest odd radix, if any
+    // Lines per workgroup. A plan with a matrix stage takes up to 16 lines, 16-column tiles of
+    // the products (and 128-byte runs of a column load), but keeps about 512 workgroups, and 16
+    // KiB a buffer set leaves several workgroups on a CU.
+    int G = std::max(1, std::min(16, 1024 / L));
+    if (odd >= kAxisMatrixMin) {
+      const long long lines = (long long)g.nlines * nplanes;
+      G = int(std::min<long long>(16, std::max<long long>(4, lines / 512)));
+      while (G > 1 && 4 * size_t(G) * (L + 1) * sizeof(T) > 40 * 1024) --G;
+    }
     const int Lp = G > 1 ? L + 1 : L;
-    const size_t lds = 4 * size_t(G) * Lp * sizeof(T);
+    size_t lds = 4 * size_t(G) * Lp * sizeof(T);
+    pl.table = odd >= kAxisMatrixMin && lds + 2 * size_t(odd) * sizeof(T) <= 64 * 1024 ? odd : 0;
+    lds += 2 * size_t(pl.table) * sizeof(T);
     hipLaunchKernelGGL((k_axis_fft<T, LOAD, STORE>), dim3((g.nlines + G - 1) / G, nplanes),
                        dim3(kAxisThreads), lds, stream_, in, out, fo_tw_[axis].as<cplx<T>>(), pl,
                        int(inverse), g, G, ph, scale);

@@ -11,7 +11,8 @@
 //   out[o] = Σ_b in[j + b·L/R]·w^(b·((j mod Ns) + a·Ns)·L/(Ns·R)),
 //   a = (o/Ns) mod R, j = (o/(Ns·R))·Ns + o mod Ns, w = exp(−2πi/L)
 // (the butterfly of Govindaraju et al., SC 2008, one output per thread, so any radix runs the
-// same code). Inverse transforms conjugate in and out; none is normalised.
+// same code), or, for an odd radix of at least kAxisMatrixMin, as matrix products
+// (axis_matrix_stage). Inverse transforms conjugate in and out; none is normalised.
 #pragma once
 
 #include "cplx.hpp"
@@ -22,8 +23,12 @@ constexpr int kAxisMaxStages = 24;
 constexpr int kAxisMax = 4096;   // longest object side the transforms take
 constexpr int kAxisThreads = 256;
 
+// Odd radices from here on run as matrix products (3 stays a butterfly: 1 of 16 rows used).
+constexpr int kAxisMatrixMin = 5;
+
+// `table`: the largest radix whose cos/sin table has room in a launch's LDS (0: none).
 struct AxisPlan {
-  int L, nst;
+  int L, nst, table;
   int radix[kAxisMaxStages];
 };
 
@@ -63,9 +68,105 @@ __device__ __forceinline__ double2 sample_phase(double2 t, int jy, int jx, int n
   return make_double2(c, s);
 }
 
+// A 16×16 += 16×4·4×16 matrix-core product in the element type: lane l holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and of the result column l % 16, rows row(l, 0 .. 3).
+template <typename T>
+struct AxisMfma;
+template <>
+struct AxisMfma<float> {
+  using V = float __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ V mac(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+template <>
+struct AxisMfma<double> {
+  using V = double __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ V mac(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
+};
+
+// Stage of odd radix R over the workgroup's G lines (nbf = G·L/R butterflies), as two real matrix
+// products. The twiddled inputs y_b of a butterfly fold into s_b = y_b + y_(R−b) and d_b = y_b −
+// y_(R−b), b = 1 .. h, h = (R − 1)/2 (in place in the source buffers), and
+//   X_a, X_(R−a) = y_0 + P_a ∓ i·Q_a,  P_a = Σ_b cos(2πab/R)·s_b,  Q_a = Σ_b sin(2πab/R)·d_b
+// for a = 0 .. h: a quarter of the direct sum's products, and contractions of a fixed (h + 1) × h
+// matrix with the butterflies' real and imaginary parts as columns, which the matrix cores take in
+// the element type (the products' inputs and sums stay 32 or 64 bits). The direct form spent its
+// time on one gathered twiddle, two LDS words and an index update per product. `tab`: 2·R values.
+// 158-pixel object sides (2·79), 32 windows of 128², complex64, a column pass: 74 µs before.
+template <typename T>
+__device__ __forceinline__ void axis_matrix_stage(int L, int Lp, int G, int R, int Ns,
+                                                  const cplx<T>* __restrict__ tw, T* sre, T* sim,
+                                                  T* dre, T* dim, T* tab) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int LR = L / R, NR = Ns * R, h = (R - 1) / 2, nbf = G * LR;
+  for (int t = tid; t < R; t += kAxisThreads) {
+    const cplx<T> w = ld(tw + t * LR);
+    tab[t] = w.x;
+    tab[R + t] = -w.y;
+  }
+  for (int idx = tid; idx < nbf * h; idx += kAxisThreads) {
+    const int bf = idx % nbf, b = idx / nbf + 1;
+    const int gi = bf / LR, j = bf % LR;
+    const int p = gi * Lp + j + b * LR, m = gi * Lp + j + (R - b) * LR;
+    cplx<T> u{sre[p], sim[p]}, v{sre[m], sim[m]};
+    if (Ns > 1) {
+      const int base = (j % Ns) * (L / NR);
+      u = u * ld(tw + (b * base) % L);
+      v = v * ld(tw + ((R - b) * base) % L);
+    }
+    sre[p] = u.x + v.x;
+    sim[p] = u.y + v.y;
+    sre[m] = u.x - v.x;
+    sim[m] = u.y - v.y;
+  }
+  __syncthreads();
+  using F = AxisMfma<T>;
+  const int nct = (2 * nbf + 15) / 16, nrt = h / 16 + 1;
+  // A wave's tasks are 16 × 16 tiles of the result; every lane runs every product.
+  for (int task = wave; task < nct * nrt; task += kAxisThreads / 64) {
+    const int ctile = task % nct, rtile = task / nct;
+    const int col = ctile * 16 + (lane & 15), im = col & 1;
+    const bool in = col < 2 * nbf;
+    const int bf = in ? col >> 1 : 0;
+    const int gi = bf / LR, j = bf % LR;
+    const T* x = (im ? sim : sre) + gi * Lp + j;
+    const int a = rtile * 16 + (lane & 15), k = lane >> 4;
+    typename F::V P = {0, 0, 0, 0}, Q = {0, 0, 0, 0};
+    int t = int((long long)a * (k + 1) % R);
+    const int dt = 4 * a % R;
+    for (int b0 = 1; b0 <= h; b0 += 4) {
+      const int b = b0 + k, bc = b <= h ? b : h;  // past h: a zero row times a finite value
+      const T c = b <= h ? tab[t] : T(0), sn = b <= h ? tab[R + t] : T(0);
+      P = F::mac(c, x[bc * LR], P);
+      Q = F::mac(sn, x[(R - bc) * LR], Q);
+      t += dt;
+      if (t >= R) t -= R;
+    }
+    const T y0 = x[0];
+    T* out = (im ? dim : dre) + gi * Lp + (j / Ns) * NR + j % Ns;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const T qo = __shfl_xor(Q[r], 1, 64);  // the other component's Q
+      const T qs = im ? -qo : qo, y = y0 + P[r];
+      const int ar = rtile * 16 + F::row(lane, r);
+      if (in && ar <= h) {
+        out[ar * Ns] = y + qs;
+        if (ar > 0) out[(R - ar) * Ns] = y - qs;
+      }
+    }
+  }
+  __syncthreads();
+}
+
 // One pass of line transforms over planes. Grid (ceil(nlines/G), nplanes), kAxisThreads
-// threads, dynamic LDS 4·G·Lp·sizeof(T) (Lp = L + 1 when G > 1, so that a column load's lanes
-// fall on different banks).
+// threads, dynamic LDS (4·G·Lp + 2·plan.table)·sizeof(T) (Lp = L + 1 when G > 1, so that a column
+// load's lanes fall on different banks).
 template <typename T, int LOAD, int STORE>
 __global__ __launch_bounds__(kAxisThreads) void k_axis_fft(const cplx<T>* __restrict__ in,
                                                            void* __restrict__ out,
@@ -79,6 +180,7 @@ __global__ __launch_bounds__(kAxisThreads) void k_axis_fft(const cplx<T>* __rest
   T* im0 = re0 + G * Lp;
   T* re1 = im0 + G * Lp;
   T* im1 = re1 + G * Lp;
+  T* tab = im1 + G * Lp;
   const int p = blockIdx.y;
   const int l0 = blockIdx.x * G;
   const int gl = g.nlines - l0 < G ? g.nlines - l0 : G;
@@ -123,7 +225,9 @@ __global__ __launch_bounds__(kAxisThreads) void k_axis_fft(const cplx<T>* __rest
   for (int s = 0; s < plan.nst; ++s) {
     const int R = plan.radix[s];
     const int LR = L / R, NR = Ns * R, stride = L / NR;
-    for (int idx = threadIdx.x; idx < tot; idx += kAxisThreads) {
+    const bool matrix = R >= kAxisMatrixMin && R <= plan.table;
+    if (matrix) axis_matrix_stage(L, Lp, G, R, Ns, tw, sre, sim, dre, dim, tab);
+    for (int idx = threadIdx.x; idx < tot && !matrix; idx += kAxisThreads) {
       const int gi = idx / L, o = idx % L;
       const int a = (o / Ns) % R, j = (o / NR) * Ns + o % Ns;
       const int base = ((j % Ns) + a * Ns) * stride;  // < L
@@ -142,7 +246,7 @@ __global__ __launch_bounds__(kAxisThreads) void k_axis_fft(const cplx<T>* __rest
       dre[gi * Lp + o] = sr;
       dim[gi * Lp + o] = si;
     }
-    __syncthreads();
+    if (!matrix) __syncthreads();
     T* x = sre; sre = dre; dre = x;
     x = sim; sim = dim; dim = x;
     Ns *= R;

@@ -31,7 +31,7 @@ def scan(case):
     cy, cx = sim.corners(y, x, pixel, side, n)
     intensity = sim.intensities(obj, probe, cy, cx, sim.quad_phase(n))
     s = 2e5 / intensity.sum(axis=(1, 2)).mean()
-    start = np.exp(1j * rng.uniform(-1.0, 1.0, side))
+    start = np.exp(1j * rng.uniform(-1.0, 1.0, obj.shape))
     return dict(counts=rng.poisson(intensity * s).astype(np.float32), y=y, x=x, obj=start,
                 probe=probe * math.sqrt(s) * 0.9)
 
