@@ -25,7 +25,9 @@ def scan(case):
     n, modes, frames, side = case
     pixel = sim.pixel_size(n)
     rng = np.random.default_rng(11)
-    y, x = (rng.uniform(-(s - n) / 2 + 4, (s - n) / 2 - 4, frames) * pixel for s in side)
+    y, x = rng.uniform(-1, 1, (2, frames))
+    y, x = (v - v.mean() for v in (y, x))  # the scan is centred on its mean
+    y, x = (v / np.abs(v).max() * ((s - n) / 2 - 4) * pixel for v, s in zip((y, x), side))
     obj = sim.random_object(*side, 3)
     probe = sim.hermite_gauss_probe(n, powers=[0.8, 0.2, 0.05][:modes])
     cy, cx = sim.corners(y, x, pixel, side, n)
