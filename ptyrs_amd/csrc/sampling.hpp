@@ -97,7 +97,9 @@ struct AxisMfma<double> {
 // matrix with the butterflies' real and imaginary parts as columns, which the matrix cores take in
 // the element type (the products' inputs and sums stay 32 or 64 bits). The direct form spent its
 // time on one gathered twiddle, two LDS words and an index update per product. `tab`: 2·R values.
-// 158-pixel object sides (2·79), 32 windows of 128², complex64, a column pass: 74 µs before.
+// Against 64 bits its error is below the direct sum's (radix 79: 1.2e-7 against 1.7e-7 of the
+// norm). 158-pixel sides (2·79), 32 windows of 128², complex64: a row pass 48 → 14 µs, a window
+// column pass (its FP64 phases included) 74 → 28 µs.
 template <typename T>
 __device__ __forceinline__ void axis_matrix_stage(int L, int Lp, int G, int R, int Ns,
                                                   const cplx<T>* __restrict__ tw, T* sre, T* sim,
