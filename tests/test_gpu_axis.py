@@ -19,8 +19,8 @@ SIDES = [(64, 64), (48, 50), (49, 56), (55, 66), (62, 74), (75, 70), (61, 63)]
 @pytest.mark.parametrize("side", SIDES)
 def test_sampled_windows_at_every_plan(side, dtype, tol):
     d = small_scan(n=32, nprobe=2, npos=9, masked=False)
+    d["y"], d["x"] = d["y"] * 0.4, d["x"] * 0.4  # the frames stay inside every side
     rng = np.random.default_rng(2)
-    assert d["obj"].shape[-1] <= min(side)  # the frames stay inside
     d["obj"] = np.exp(1j * rng.uniform(-1.0, 1.0, (1, *side)))
     d0 = rng.uniform(-0.45, 0.45, (9, 2))
     g, o = gpu(d, dtype), oracle(d)
