@@ -601,6 +601,7 @@ class Engine : public EngineBase {
     ensure_lsqml(size);
     if (full_object()) fo_ensure(cap_, true);
     if (opr_on_) opr_ensure(cap_);
+    if (nslice_ == 1 && !pos_on_ && !opr_on_) csum_.ensure(sizeof(cplx<T>) * cap_ * n);
     std::vector<int> order(nepoch * nframe_);
     std::vector<std::vector<std::pair<int, int>>> spans(nepoch);
     for (size_t ic = 0; ic < nepoch; ++ic) {
@@ -807,18 +808,23 @@ class Engine : public EngineBase {
     const size_t stack = std::min<size_t>(nframe_, stack_size_ ? stack_size_ : kDefaultStack);
     ensure_workspace(stack, 1);
     const size_t nb_all = nframe_;
-    // psi_f16 holds DM's and RAAR's carried waves as f16 pairs (AP's stay complex).
-    const bool half = psi_f16_ && p.algorithm != PTYRS_AP;
+    // psi_f16 holds DM's and RAAR's carried waves as f16 pairs. AP carries none: its object
+    // update reads each frame's terms summed over the modes (csum_).
+    const bool ap = p.algorithm == PTYRS_AP;
+    const bool half = psi_f16_ && !ap;
     DevBuf& cbuf = half ? carried16_ : carried_;
     DevBuf& ibuf = half ? iter16_ : iter_;
     const size_t wbytes = half ? sizeof(uint32_t) : sizeof(cplx<T>);
-    cbuf.ensure(wbytes * nb_all * M_ * n);
+    if (ap)
+      csum_.ensure(sizeof(cplx<T>) * nb_all * n);
+    else
+      cbuf.ensure(wbytes * nb_all * M_ * n);
     if (p.algorithm == PTYRS_RAAR) ibuf.ensure(wbytes * nb_all * M_ * n);
     const int nt = ntiles();
     list_all_.ensure(sizeof(int) * size_t(nt) * nb_all);
     count_all_.ensure(sizeof(int) * size_t(nt));
     const int nstack = int((nb_all + stack - 1) / stack);
-    const int chunk = chunk_of(int(stack));
+    const int chunk = ap ? chunk_of_m(int(stack)) : chunk_of(int(stack));
     const int nchunk = int((stack + chunk - 1) / chunk);
     pnum_part_.ensure(sizeof(cplx<T>) * size_t(nstack) * nchunk * M_ * n);
     pden_part_.ensure(sizeof(T) * size_t(nstack) * nchunk * n);
@@ -856,13 +862,21 @@ class Engine : public EngineBase {
         mix.c0 = T(1.0 - 0.5 * p.mix);
         mix.c1 = T(0.5 * p.mix);
       }
-      const bool ap_probe = p.algorithm == PTYRS_AP && p.upd_probe;
+      const bool ap_probe = ap && p.upd_probe;
       for (int s = 0; s < nstack; ++s) {
         const int f0 = int(s * stack);
         const int nb = std::min<int>(int(stack), int(nframe_) - f0);
         const int* ord = iota_.as<int>() + f0;
         pass_a(ord, nb, false, mix);
         pass_b<B_AMPLITUDE>(ord, nb);
+        if (ap) {
+          pass_c_sum<false>(ord, nb, nullptr, ap_probe, csum_.as<cplx<T>>(), true,
+                            pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
+                            pden_part_.as<T>() + size_t(s) * nchunk * n);
+          const int ck = chunk_of_m(nb), nck = (nb + ck - 1) / ck;
+          if (ap_probe && nck < nchunk) zero_partials(s, nck, nchunk);
+          continue;
+        }
         const int ck = chunk_of(nb);
         const int nck = (nb + ck - 1) / ck;
         const bool dm = p.algorithm == PTYRS_DM && !first;
@@ -870,15 +884,14 @@ class Engine : public EngineBase {
           hipLaunchKernelGGL((k_pass_c_proj<T, N, H>), dim3(SR::NBLK, M_, nck), dim3(SR::NT), 0,
                              stream_, psi_.as<cplx<T>>(), cw, O_.as<cplx<T>>(), int(nxo_),
                              Wt_.as<cplx<T>>(), q_.as<cplx<T>>(), corner_.as<int2>(), ord, nb,
-                             M_, ck, int(dm), T(2.0 - p.mix), T(1.0 - p.mix), int(ap_probe),
-                             pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
-                             pden_part_.as<T>() + size_t(s) * nchunk * n, tw_.as<cplx<T>>());
+                             M_, ck, int(dm), T(2.0 - p.mix), T(1.0 - p.mix), 0,
+                             (cplx<T>*)nullptr, (T*)nullptr, tw_.as<cplx<T>>());
         });
-        if (ap_probe && nck < nchunk) zero_partials(s, nck, nchunk);
       }
       const int tot_chunks = nstack * nchunk;
-      if (p.algorithm == PTYRS_AP) {
-        if (p.upd_obj) object_blend(p.obj_inertia, cw);
+      if (ap) {
+        if (p.upd_obj)
+          object_blend(p.obj_inertia, Carried<T, false>{csum_.as<cplx<T>>()}, true);
         if (p.upd_probe) probe_blend(tot_chunks, p.probe_inertia);
       } else {
         for (size_t l = 0; l < p.loops; ++l) {
@@ -1440,14 +1453,14 @@ class Engine : public EngineBase {
     ensure_workspace(stack, 1);
     const size_t no = nobj_ * nyo_ * nxo_, np = nprobe_ * n;
     const int nt = ntiles();
-    carried_.ensure(sizeof(cplx<T>) * nframe_ * M_ * n);
+    csum_.ensure(sizeof(cplx<T>) * nframe_ * n);
     psi3_.ensure(sizeof(cplx<T>) * 3 * stack * M_ * n);
     for (DevBuf* b : {&gO_, &hO_, &dOc_}) b->ensure(sizeof(cplx<T>) * no);
     for (DevBuf* b : {&gP_, &hP_, &dPc_, &dWt_}) b->ensure(sizeof(cplx<T>) * np);
     list_all_.ensure(sizeof(int) * size_t(nt) * nframe_);
     count_all_.ensure(sizeof(int) * size_t(nt));
     const int nstack = int((nframe_ + stack - 1) / stack);
-    const int chunk = chunk_of(int(stack));
+    const int chunk = chunk_of_m(int(stack));
     const int nchunk = int((stack + chunk - 1) / chunk);
     pnum_part_.ensure(sizeof(cplx<T>) * size_t(nstack) * nchunk * M_ * n);
     pden_part_.ensure(sizeof(T) * size_t(nstack) * nchunk * n);
@@ -1497,25 +1510,18 @@ class Engine : public EngineBase {
         const int* ord = iota_.as<int>() + f0;
         pass_a(ord, nb, false);
         pass_b<B_GRAD>(ord, nb);
-        const int ck = chunk_of(nb);
-        const int nck = (nb + ck - 1) / ck;
-        run(K_PASS_C, [&] {
-          hipLaunchKernelGGL((k_pass_c_proj<T, N, false>), dim3(SR::NBLK, M_, nck),
-                             dim3(SR::NT), 0, stream_, psi_.as<cplx<T>>(),
-                             Carried<T, false>{carried_.as<cplx<T>>()}, O_.as<cplx<T>>(),
-                             int(nxo_), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
-                             corner_.as<int2>(), ord, nb, M_, ck, 0, T(0), T(0), int(up),
-                             pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
-                             pden_part_.as<T>() + size_t(s) * nchunk * n, tw_.as<cplx<T>>());
-        });
+        pass_c_sum<false>(ord, nb, nullptr, up, csum_.as<cplx<T>>(), true,
+                          pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
+                          pden_part_.as<T>() + size_t(s) * nchunk * n);
+        const int ck = chunk_of_m(nb), nck = (nb + ck - 1) / ck;
         if (up && nck < nchunk) zero_partials(s, nck, nchunk);
       }
       if (uo) {
         run(K_OBJ_UPDATE, [&] {
-          obj_dir(gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), carried_.as<cplx<T>>(), N,
-                             M_, corner_.as<int2>(), iota_.as<int>(), list_all_.as<int>(),
-                             count_all_.as<int>(), int(nframe_), int(nyo_), int(nxo_), ntx_,
-                             (const T*)nullptr, (const T*)nullptr);
+          obj_dir(gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
+                  corner_.as<int2>(), iota_.as<int>(), list_all_.as<int>(),
+                  count_all_.as<int>(), int(nframe_), int(nyo_), int(nxo_), ntx_,
+                  (const T*)nullptr, (const T*)nullptr, 0, nullptr, 0, 0, true);
         });
       }
       if (up) {
@@ -2082,6 +2088,7 @@ class Engine : public EngineBase {
                     " needs a unitary propagator; this one drops an evanescent band: only "
                     "LSQML and the LLK pass run it");
   }
+  bool exit_unitary() const { return !banded_; }
   // ... and one object slice (ptyrs/src/engine/gpu/device.rs:3100-3105).
   void one_unitary(const char* what) const {
     if (nslice_ > 1)
@@ -2874,6 +2881,7 @@ class Engine : public EngineBase {
     std::memcpy(&u, &v, sizeof u);
     return u;
   }
+  DevBuf csum_;  // per slot or frame Σ_m conj(W_m)·v_m (pass_c_sum)
   DevBuf psi_, omax_, dP_, list_, lcount_, tilemax_, pmax_, order_, llk_part_, D_;
 
   void upload_complex(DevBuf& d, const double* src, size_t count) {
@@ -3591,6 +3599,7 @@ class Engine : public EngineBase {
   void lsqml_batch(const ptyrs_lsqml_params& p, const int* ord, int nb, int off) {
     const int nt = ntiles();
     const bool gauss = p.cost == PTYRS_AMPLITUDE;
+    const bool linear = !gauss && exit_unitary();
     run(K_BIN, [&] {
       bin_tiles(corner_.as<int2>(), ord, nb, N, ntx_, int(cap_), list_.as<int>(),
                          lcount_.as<int>(), (const T*)nullptr, M_, int(nyo_), int(nxo_),
@@ -3607,7 +3616,10 @@ class Engine : public EngineBase {
         hipLaunchKernelGGL(k_lsqml_prev<T>, dim3(1), dim3(THREADS), 0, stream_,
                            afar_all_.as<T>(), ord, nb, prev_.as<T>());
       });
-      pass_b<B_ICALC>(ord, nb, ba);
+      if (linear)
+        pass_b<B_XI>(ord, nb, ba);
+      else
+        pass_b<B_ICALC>(ord, nb, ba);
       run(K_OTHER, [&] {
         hipLaunchKernelGGL(k_lsqml_xi<T>, dim3(1), dim3(THREADS), 0, stream_,
                            xi_part_.as<double>(), int(SB::NBLK), nb, prev_.as<T>(),
@@ -3619,25 +3631,21 @@ class Engine : public EngineBase {
                            xi_part2_.as<double>(), xb, nb, prev_.as<T>() + 1, afar_tmp_.as<T>(),
                            (T*)nullptr);
       });
-      pass_b<B_POISSON>(ord, nb, ba);
+      if (!linear) pass_b<B_POISSON>(ord, nb, ba);
     }
     run(K_OTHER, [&] {
       hipLaunchKernelGGL(k_lsqml_log_afar<T>, dim3((nb + 255) / 256), dim3(256), 0, stream_,
                          afar_tmp_.as<T>(), ord, nb, afar_all_.as<T>(),
                          log_.as<double>() + 3 * size_t(off), int(gauss), 3);
     });
-    const int chunk = chunk_of(nb);
+    pass_c_sum<true>(ord, nb, linear ? (const T*)afar_tmp_.as<T>() : nullptr, true,
+                     csum_.as<cplx<T>>(), false, dP_.as<cplx<T>>(), nullptr);
+    const int chunk = chunk_of_m(nb);
     const int nchunk = (nb + chunk - 1) / chunk;
-    run(K_PASS_C, [&] {
-      hipLaunchKernelGGL((k_pass_c_chi<T, N>), dim3(SR::NBLK, M_, nchunk), dim3(SR::NT), 0,
-                         stream_, psi_.as<cplx<T>>(), O_.as<cplx<T>>(), int(nxo_),
-                         Wt_.as<cplx<T>>(), q_.as<cplx<T>>(), corner_.as<int2>(), ord, nb, M_,
-                         chunk, 1, dP_.as<cplx<T>>(), tw_.as<cplx<T>>());
-    });
     run(K_OBJ_DIR, [&] {
-      obj_dir(dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
-                         corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
-                         int(nyo_), int(nxo_), ntx_, pre_.as<T>(), floor_.as<T>());
+      obj_dir(dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
+              corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_), int(nyo_),
+              int(nxo_), ntx_, pre_.as<T>(), floor_.as<T>(), 0, nullptr, 0, 0, true);
     });
     const int total = int(nprobe_ * n);
     const int xb = aux_blocks();
@@ -4043,7 +4051,7 @@ class Engine : public EngineBase {
 
   // Object update of AP/DM/RAAR: tile lists over every frame, norm = Σ_m D_m, its max, blend.
   template <bool H>
-  void object_blend(double inertia, Carried<T, H> cw) {
+  void object_blend(double inertia, Carried<T, H> cw, bool summed = false) {
     const int nt = ntiles();
     run(K_BIN, [&] {
       norm2_planes();
@@ -4061,7 +4069,7 @@ class Engine : public EngineBase {
       obj_blend<H>(O_.as<cplx<T>>(), Wt_.as<cplx<T>>(), D_.as<T>(), cw, N, M_,
                          corner_.as<int2>(), iota_.as<int>(),
                          list_all_.as<int>(), count_all_.as<int>(), int(nframe_), int(nyo_),
-                         int(nxo_), ntx_, pmax_.as<T>(), T(inertia));
+                         int(nxo_), ntx_, pmax_.as<T>(), T(inertia), 0, summed);
     });
   }
 
@@ -4157,15 +4165,37 @@ class Engine : public EngineBase {
     else
       f(std::integral_constant<int, 1>{});
   }
-  // Modes whose loads the tile gathers issue together: 1, 2 or (3 and more) 4.
+  // Modes whose loads the tile gathers issue together: 1, 2 or (3 and more) 4; 0 for planes that
+  // hold the modes' sums.
   template <typename F>
-  void mode_chunk(F&& f) {
-    if (M_ == 1)
+  void mode_chunk(bool summed, F&& f) {
+    if (summed)
+      f(std::integral_constant<int, 0>{});
+    else if (M_ == 1)
       f(std::integral_constant<int, 1>{});
     else if (M_ == 2)
       f(std::integral_constant<int, 2>{});
     else
       f(std::integral_constant<int, 4>{});
+  }
+  // Pass C with the modes' terms summed over `nb` slots into `sums` (plane order[b] with
+  // by_frame, else b), chunk_of_m(nb) slots a chunk.
+  template <bool CHI>
+  void pass_c_sum(const int* ord, int nb, const T* a_far, bool probe_dir, cplx<T>* sums,
+                  bool by_frame, cplx<T>* num_part, T* den_part) {
+    const int chunk = chunk_of_m(nb);
+    const int nchunk = (nb + chunk - 1) / chunk;
+    run(K_PASS_C, [&] {
+      with_modes([&](auto mm) {
+        constexpr int MM = decltype(mm)::value;
+        constexpr int G = rows_per_group(N, SR::L, MM);
+        hipLaunchKernelGGL((k_pass_c_sum<T, N, MM, CHI>), dim3(N / G, nchunk),
+                           dim3(pass_c_sum_threads<T, N, MM>()), 0, stream_, psi_.as<cplx<T>>(),
+                           O_.as<cplx<T>>(), int(nxo_), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
+                           corner_.as<int2>(), ord, nb, chunk, a_far, int(probe_dir), sums,
+                           int(by_frame), num_part, den_part, tw_.as<cplx<T>>());
+      });
+    });
   }
   // Workgroups of k_probe_apply and k_probe_mean.
   static unsigned chunk_blocks(int total, int nchunk) {
@@ -4185,9 +4215,10 @@ class Engine : public EngineBase {
   void obj_dir(cplx<T>* dO, const cplx<T>* Wt, const cplx<T>* chi, int side, int M,
                const int2* corner, const int* ord, const int* list, const int* count, int cap,
                int nyo, int nxo, int ntx, const T* pre, const T* floor, int per_view = 0,
-               const cplx<T>* q = nullptr, int q_frame = 0, int accumulate = 0) {
+               const cplx<T>* q = nullptr, int q_frame = 0, int accumulate = 0,
+               bool summed = false) {
     split_tiles([&](auto sp) {
-      mode_chunk([&](auto mm) {
+      mode_chunk(summed, [&](auto mm) {
         constexpr int SP = decltype(sp)::value, MM = decltype(mm)::value;
         hipLaunchKernelGGL((k_lsqml_obj_dir<T, SP, MM>), dim3(ntiles()), dim3(THREADS * SP), 0,
                            stream_, dO, Wt, chi, side, M, corner, ord, list, count, cap, nyo,
@@ -4198,9 +4229,10 @@ class Engine : public EngineBase {
   template <bool H>
   void obj_blend(cplx<T>* O, const cplx<T>* Wt, const T* D, Carried<T, H> cw, int side, int M,
                  const int2* corner, const int* ord, const int* list, const int* count, int cap,
-                 int nyo, int nxo, int ntx, const T* nmax, T inertia, int w_view = 0) {
+                 int nyo, int nxo, int ntx, const T* nmax, T inertia, int w_view = 0,
+                 bool summed = false) {
     split_tiles([&](auto sp) {
-      mode_chunk([&](auto mm) {
+      mode_chunk(summed, [&](auto mm) {
         constexpr int SP = decltype(sp)::value, MM = decltype(mm)::value;
         hipLaunchKernelGGL((k_obj_blend<T, H, SP, MM>), dim3(ntiles()), dim3(THREADS * SP), 0,
                            stream_, O, Wt, D, cw, side, M, corner, ord, list, count, cap, nyo,

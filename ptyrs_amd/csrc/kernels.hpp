@@ -287,15 +287,15 @@ __global__ __launch_bounds__((RowShape<T, N>::NT)) void k_pass_a(
 
 // ---- pass B: column transforms, the detector-plane operator, inverse column transforms --------
 enum PassB { B_RPIE = 0, B_LLK = 1, B_AMPLITUDE = 2, B_GAUSS = 3, B_ICALC = 4, B_POISSON = 5,
-             B_GRAD = 6, B_GRAD_AMP = 7, B_BH = 8 };
+             B_GRAD = 6, B_GRAD_AMP = 7, B_BH = 8, B_XI = 9 };
 
 // Per-slot values some pass-B modes read or write.
 template <typename T>
 struct BArgs {
   const T* a_far;   // B_POISSON: LSQML far-field step per batch slot
-  const T* prev;    // B_ICALC: batch mean of the slots' last a_far
-  double* part;     // B_ICALC: per-workgroup (num, den) of the Poisson xi solver
-  T* icalc;         // B_ICALC: model intensity per slot and pixel, DFT index order
+  const T* prev;    // B_ICALC, B_XI: batch mean of the slots' last a_far
+  double* part;     // B_ICALC, B_XI: per-workgroup (num, den) of the Poisson xi solver
+  T* icalc;         // B_ICALC, B_XI: model intensity per slot and pixel, DFT index order
   cplx<T>* keep = nullptr;  // B_BH: the detector-plane field U·ψ per view ([slot·M + m][n])
 };
 
@@ -326,7 +326,10 @@ constexpr int pass_b_threads() {
 // B_GAUSS and B_POISSON scale the field by (1 − a_far·c)/n with LSQML's residual c (Gaussian
 // 2(1 − √iobs/(√icalc + 1e-9)) with a_far = 1/2, Poisson 1 − iobs/(icalc + 1e-6)), 0 where
 // masked (ptyrs/src/engine/lsqml.rs:97-170). B_ICALC stores icalc and the first pass of the
-// Poisson a_far solver's sums and stores no field.
+// Poisson a_far solver's sums and stores no field. B_XI does the same and scales the field by the
+// Poisson c/n: where the exit transform U is unitary, ψ' − ψ = −a_far·Uᴴ(c·Uψ), so a_far can
+// follow in pass C and the field need not be transformed a second time once the solver has it
+// (256² × 4 modes, batches of 100, complex64: B_ICALC + B_POISSON 59 + 80 µs, B_XI 103 µs).
 // ROW = false: lines are columns (the far field's column pass); ROW = true: lines are rows (the
 // angular spectrum's second row pass). `norm` is 1/n (one unnormalised DFT round trip) or 1/n²
 // (two).
@@ -398,7 +401,8 @@ __global__ __launch_bounds__((pass_b_threads<T, N, M>())) void k_pass_b(
   T afar = 0;
   double prev = 0;
   if constexpr (MODE == B_POISSON) afar = ba.a_far[b];
-  if constexpr (MODE == B_ICALC) prev = double(ba.prev[0]);
+  constexpr bool XI = MODE == B_ICALC || MODE == B_XI;
+  if constexpr (XI) prev = double(ba.prev[0]);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     if (e % M != m) continue;
@@ -444,10 +448,11 @@ __global__ __launch_bounds__((pass_b_threads<T, N, M>())) void k_pass_b(
         else c = T(1) - T(io) / (ic + T(1e-6));
       }
       r = (T(1) - (MODE == B_GAUSS ? T(0.5) : afar) * c) * inv_n;
-    } else if constexpr (MODE == B_ICALC) {
+    } else if constexpr (XI) {
       const T ic = I * inv_n;
       ba.icalc[(size_t)b * n + at(e)] = ic;
       if (io >= 0.f) {
+        r = (T(1) - T(io) / (ic + T(1e-6))) * inv_n;
         const double yp = double(ic), yt = double(io);
         const double xi = 1.0 - yt / (yp + 1e-5);
         acc[0] += xi * (yp - yt / (1.0 - prev * xi));
@@ -473,14 +478,16 @@ __global__ __launch_bounds__((pass_b_threads<T, N, M>())) void k_pass_b(
       double s = block_reduce<NT>(acc[i], red, AddOp());
       if (tid == 0) llk_part[((size_t)f * S::NBLK + bxy.x) * 4 + i] = s;
     }
-  } else if constexpr (MODE == B_ICALC) {
+  }
+  if constexpr (XI) {
     __shared__ double red[NT];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       double s = block_reduce<NT>(acc[i], red, AddOp());
       if (tid == 0) ba.part[((size_t)b * S::NBLK + bxy.x) * 2 + i] = s;
     }
-  } else {
+  }
+  if constexpr (MODE != B_LLK && MODE != B_ICALC) {
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = v[e] * lim[key(e)];
@@ -750,6 +757,122 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_rpie
 #pragma unroll
     for (int e = 0; e < E; ++e)
       st(out + jl + TL * e, cmulc(ld(q + (size_t)y * N + jl + TL * e), acc[e]));
+  }
+}
+
+// Pass C with the modes' object terms summed, in k_pass_c_rpie_sum's shape (M groups of G rows,
+// the terms in LDS, added over the modes one slot later). Per slot each group transforms its rows
+// back to x, takes the field v of its mode, and the slot's Σ_m conj(W_m)·v_m goes to one plane of
+// `sums` (plane order[b] with by_frame, else b), so that the object update reads one plane a slot
+// instead of M fields and M probe terms. With `probe_dir` conj(O·q)·v and (den_part not null)
+// |O|² are added into per-chunk partials.
+//   CHI (LSQML): v = χ, stored over the projected field: −a_far[b]·x of B_XI's x, or with a_far
+//   null x − W·O.
+//   otherwise (AP's projected waves, ML's gradient): v = x, which is stored nowhere else.
+// 256² × 4 modes complex64, 1024 frames: AP's pass C and object update took 2.97 + 2.13 ms per 3
+// cycles with every mode's wave stored and read again, 2.22 + 0.52 so; LSQML's 95 + 64 µs per 100
+// slots, 89 + 25. ptyrs/src/engine/lsqml.rs:97-228, ptyrs/src/engine/ops.rs:345-381
+template <typename T, int N, int M, bool CHI>
+__global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_sum(
+    cplx<T>* __restrict__ psi, const cplx<T>* __restrict__ O, int nxo,
+    const cplx<T>* __restrict__ Wt, const cplx<T>* __restrict__ q,
+    const int2* __restrict__ corner, const int* __restrict__ order, int nb, int chunk,
+    const T* __restrict__ a_far, int probe_dir, cplx<T>* __restrict__ sums, int by_frame,
+    cplx<T>* __restrict__ num_part, T* __restrict__ den_part, const cplx<T>* __restrict__ tw) {
+  using S = RowShapeC<T, N>;
+  constexpr int E = S::E, TL = S::TL;
+  constexpr int G = rows_per_group(N, S::L, M);
+  constexpr int n = N * N;
+  constexpr int TW = M * G * N;  // terms per buffer
+  constexpr bool FITS = M * G <= S::L;
+  constexpr int PLD = N + (N >> 4) + 1;
+  using At = std::conditional_t<FITS, typename S::AtRow, LdsPlain>;
+  constexpr int LDW = FITS ? S::LDS_WORDS : M * G * PLD;
+  __shared__ T lre[LDW], lim[LDW];
+  __shared__ cplx<T> stw[N];
+  constexpr bool DB = 2 * LDW * sizeof(T) + N * sizeof(cplx<T>) + 2 * TW * sizeof(cplx<T>) <=
+                      160 * 1024;
+  constexpr int NBUF = DB ? 2 : 1;
+  __shared__ cplx<T> terms[NBUF * TW];
+  const int tid = threadIdx.x;
+  const int m = wave_uniform<G * TL>(tid / (G * TL)), l = (tid / TL) % G, jl = tid % TL;
+  const int line = m * G + l;
+  const int y = blockIdx.x * G + l;
+  const int ch = blockIdx.y;
+  const int b0 = ch * chunk;
+  const int b1 = b0 + chunk < nb ? b0 + chunk : nb;
+  stage_twiddles<T, N, G * M * TL>(stw, tw);
+  // Every slot's transform uses the lane's twiddles, held in registers for float.
+  constexpr bool TC = sizeof(T) == 4;
+  cplx<T> twc[TC ? tw_cache_size(N, E) : 1];
+  if constexpr (TC) load_tw_cache<T, N, E>(twc, jl, stw);
+  // The partials are Kahan sums: a chunk's slots would else be a longer plain chain than a
+  // per-mode launch's shorter chunks had.
+  cplx<T> w[E];
+  kahan<T> ar[E], ai[E], den[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    w[e] = ld(Wt + (size_t)m * n + (size_t)y * N + jl + TL * e);
+  }
+  auto store_sum = [&](int sb, int buf) {
+    cplx<T>* out = sums + (size_t)(by_frame ? order[sb] : sb) * n + (size_t)y * N + jl;
+    const cplx<T>* t = terms + buf * TW + l * N + jl;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (e % M != m) continue;
+      cplx<T> sum = t[TL * e];
+#pragma unroll
+      for (int k = 1; k < M; ++k) sum = sum + t[k * G * N + TL * e];
+      st(out + TL * e, sum);
+    }
+  };
+  const int lb = FITS ? S::base_row(line) : line * PLD;
+  for (int b = b0; b < b1; ++b) {
+    cplx<T> v[E], ow[E];
+    cplx<T>* row = psi + ((size_t)(b * M + m) * N + y) * N + jl;
+    const int2 c = corner[order[b]];
+    const cplx<T>* orow = O + (size_t)(c.x + y) * nxo + c.y + jl;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      v[e] = ld(row + TL * e);
+      ow[e] = ld(orow + TL * e);
+    }
+    const T gain = CHI && a_far ? -a_far[b] : T(1);
+    // The transform's barriers also order the previous slot's term writes before the reads
+    // below, and this slot's reads of buffer (b − 1) before the writes of slot b + 1.
+    line_fft<T, N, E, true, At, TC>(v, jl, lre + lb, lim + lb, stw, twc);
+    if (b > b0) {
+      store_sum(b - 1, DB ? (b - 1) & 1 : 0);
+      if constexpr (!DB) __syncthreads();
+    }
+    cplx<T>* trow = terms + (DB ? b & 1 : 0) * TW + line * N + jl;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if constexpr (CHI) {
+        v[e] = a_far ? v[e] * gain : v[e] - w[e] * ow[e];
+        st(row + TL * e, v[e]);
+      }
+      trow[TL * e] = cmulc(w[e], v[e]);
+      if (probe_dir) {
+        const cplx<T> d = cmulc(ow[e], v[e]);
+        ar[e].add(d.x);
+        ai[e].add(d.y);
+        if constexpr (!CHI) den[e].add(norm2(ow[e]));
+      }
+    }
+  }
+  if (b1 > b0) {
+    __syncthreads();
+    store_sum(b1 - 1, DB ? (b1 - 1) & 1 : 0);
+  }
+  if (probe_dir) {
+    const size_t row = (size_t)y * N + jl;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      st(num_part + ((size_t)ch * M + m) * n + row + TL * e, cmulc(ld(q + row + TL * e), cplx<T>{ar[e].s, ai[e].s}));
+      if constexpr (!CHI)
+        if (m == 0) den_part[(size_t)ch * n + row + TL * e] = den[e].s;
+    }
   }
 }
 
@@ -1178,7 +1301,8 @@ __global__ __launch_bounds__(THREADS) void k_lsqml_xi_sums(
 // Σ_m Σ_views conj(W·q)·χ_m (Kahan-compensated) and divides by √(pre² + floor); 0 where no view
 // covers it. W is W_m ([M][n]) or, with per_view, the slot's own plane ([slot·M + m][n], a
 // multislice slice's incident waves or a moved probe); q (nullable) a plane phase, per slot
-// ([slot][n]) with q_frame. With `accumulate` the result is added to dO.
+// ([slot][n]) with q_frame. With `accumulate` the result is added to dO. MM = 0: `chi` holds the
+// modes' sums already ([slot][n], k_pass_c_sum), which are only added.
 // ptyrs/src/engine/lsqml.rs:183-188, :587-598; ptyrs/src/engine/ops.rs:279-310;
 // ptyrs/src/engine/multislice.rs:402-430
 template <typename T, int SP, int MM>
@@ -1205,7 +1329,7 @@ __global__ __launch_bounds__(THREADS * SP) void k_lsqml_obj_dir(
     }
     __syncthreads();
     // SU slots of MM modes per step: their loads are issued together, then added in slot order.
-    constexpr int SU = 4 / MM;
+    constexpr int SU = MM > 0 ? 4 / MM : 4;
     const int2 sh = share_of<SP>(g, k);
     for (int i0 = sh.x; i0 < sh.y && X < nxo; i0 += SU) {
       int j[SU];
@@ -1218,15 +1342,29 @@ __global__ __launch_bounds__(THREADS * SP) void k_lsqml_obj_dir(
         const int x = X - cs[i].z, y = Y - cs[i].y;
         ok[u] = i0 + u < sh.y && x >= 0 && x < N && y >= 0 && y < N;
         j[u] = y * N + x;
-        cv[u] = (size_t)cs[i].x * M * n;
+        cv[u] = (size_t)cs[i].x * (MM > 0 ? M : 1) * n;
         if (q && ok[u]) qj[u] = ld(q + (q_frame ? (size_t)cs[i].x * n : 0) + j[u]);
       }
-      for (int m0 = 0; m0 < M; m0 += MM) {
-        cplx<T> w[SU][MM], c[SU][MM];
+      if constexpr (MM == 0) {
+        cplx<T> c[SU];
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+          if (ok[u]) c[u] = ld(chi + cv[u] + j[u]);
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+          if (ok[u]) {
+            sr.add(c[u].x);
+            si.add(c[u].y);
+          }
+        continue;
+      }
+      constexpr int MC = MM > 0 ? MM : 1;
+      for (int m0 = 0; m0 < M; m0 += MC) {
+        cplx<T> w[SU][MC], c[SU][MC];
 #pragma unroll
         for (int u = 0; u < SU; ++u)
 #pragma unroll
-          for (int m = 0; m < MM; ++m)
+          for (int m = 0; m < MC; ++m)
             if (ok[u] && m0 + m < M) {
               const size_t p = (size_t)(m0 + m) * n + j[u];
               w[u][m] = ld(Wt + (per_view ? cv[u] : 0) + p);
@@ -1235,7 +1373,7 @@ __global__ __launch_bounds__(THREADS * SP) void k_lsqml_obj_dir(
 #pragma unroll
         for (int u = 0; u < SU; ++u)
 #pragma unroll
-          for (int m = 0; m < MM; ++m)
+          for (int m = 0; m < MC; ++m)
             if (ok[u] && m0 + m < M) {
               const cplx<T> v = cmulc(q ? w[u][m] * qj[u] : w[u][m], c[u][m]);
               sr.add(v.x);
@@ -2271,7 +2409,8 @@ __global__ void k_probe_blend(cplx<T>* __restrict__ P, cplx<T>* __restrict__ Wt,
 // PyNX blend of the object from tile-owned sums over every view: every pixel owned by one thread
 // sums Σ_m Σ_views conj(W_m)·ψ_m (Kahan) in view order, and O = (num + reg·O)/max(norm + reg,
 // 1e-12) with norm = Σ_m D_m from k_bin_tiles and reg = inertia·max(norm). With w_view W is the
-// frame's own wave (plane frame·M + m of Wt, a moved probe; the order is every frame's).
+// frame's own wave (plane frame·M + m of Wt, a moved probe; the order is every frame's). MM = 0:
+// `carried` holds the modes' sums ([frame][n], k_pass_c_sum).
 template <typename T, bool H, int SP, int MM>
 __global__ __launch_bounds__(THREADS * SP) void k_obj_blend(
     cplx<T>* __restrict__ O, const cplx<T>* __restrict__ Wt, const T* __restrict__ D,
@@ -2296,7 +2435,7 @@ __global__ __launch_bounds__(THREADS * SP) void k_obj_blend(
     }
     __syncthreads();
     // SU views of MM modes per step: their loads are issued together, then added in view order.
-    constexpr int SU = 4 / MM;
+    constexpr int SU = MM > 0 ? 4 / MM : 4;
     const int2 sh = share_of<SP>(g, k);
     for (int i0 = sh.x; i0 < sh.y && inside; i0 += SU) {
       int j[SU];
@@ -2308,14 +2447,28 @@ __global__ __launch_bounds__(THREADS * SP) void k_obj_blend(
         const int y = Y - cs[i].y, x = X - cs[i].z;
         ok[u] = i0 + u < sh.y && y >= 0 && y < N && x >= 0 && x < N;
         j[u] = y * N + x;
-        cv[u] = (size_t)cs[i].x * M * n;
+        cv[u] = (size_t)cs[i].x * (MM > 0 ? M : 1) * n;
       }
-      for (int m0 = 0; m0 < M; m0 += MM) {
-        cplx<T> w[SU][MM], c[SU][MM];
+      if constexpr (MM == 0) {
+        cplx<T> c[SU];
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+          if (ok[u]) c[u] = carried.get(cv[u] + j[u]);
+#pragma unroll
+        for (int u = 0; u < SU; ++u)
+          if (ok[u]) {
+            sr.add(c[u].x);
+            si.add(c[u].y);
+          }
+        continue;
+      }
+      constexpr int MC = MM > 0 ? MM : 1;
+      for (int m0 = 0; m0 < M; m0 += MC) {
+        cplx<T> w[SU][MC], c[SU][MC];
 #pragma unroll
         for (int u = 0; u < SU; ++u)
 #pragma unroll
-          for (int m = 0; m < MM; ++m)
+          for (int m = 0; m < MC; ++m)
             if (ok[u] && m0 + m < M) {
               const size_t p = (size_t)(m0 + m) * n + j[u];
               w[u][m] = ld(Wt + (w_view ? cv[u] : 0) + p);
@@ -2324,7 +2477,7 @@ __global__ __launch_bounds__(THREADS * SP) void k_obj_blend(
 #pragma unroll
         for (int u = 0; u < SU; ++u)
 #pragma unroll
-          for (int m = 0; m < MM; ++m)
+          for (int m = 0; m < MC; ++m)
             if (ok[u] && m0 + m < M) {
               const cplx<T> v = cmulc(w[u][m], c[u][m]);
               sr.add(v.x);
