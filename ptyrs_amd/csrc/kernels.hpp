@@ -664,10 +664,11 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_rpie
   constexpr int LDW = FITS ? S::LDS_WORDS : M * G * PLD;
   __shared__ T lre[LDW], lim[LDW];
   __shared__ cplx<T> stw[N];
-  // Two term buffers (slot b in buffer b mod 2) where they fit in LDS, else one, with a
+  // Two term buffers (slot b in buffer b mod 2) for float where they fit in LDS, else one, with a
   // barrier between a slot's sums and the next slot's terms.
-  constexpr bool DB = 2 * LDW * sizeof(T) + N * sizeof(cplx<T>) + 2 * TW * sizeof(cplx<T>) <=
-                      160 * 1024;
+  constexpr bool DB = sizeof(T) == 4 && 2 * LDW * sizeof(T) + N * sizeof(cplx<T>) +
+                                                2 * TW * sizeof(cplx<T>) <=
+                                            160 * 1024;
   constexpr int NBUF = DB ? 2 : 1;
   __shared__ cplx<T> terms[NBUF * TW];
   const int tid = threadIdx.x;
@@ -678,9 +679,13 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_rpie
   const int b0 = ch * chunk;
   const int b1 = b0 + chunk < nb ? b0 + chunk : nb;
   stage_twiddles<T, N, G * M * TL>(stw, tw);
-  // Every slot's transform uses the lane's twiddles: held in registers.
-  cplx<T> twc[tw_cache_size(N, E)];
-  load_tw_cache<T, N, E>(twc, jl, stw);
+  // Every slot's transform uses the lane's twiddles: held in registers for float. For double they
+  // are 36 of 180 registers and the second term buffer is the LDS of a third workgroup on a CU:
+  // with both, 256² × 4 modes took 308 µs for 84 slots, without 189. (512² in float, two
+  // workgroups with them and three without: 599 µs against 650.)
+  constexpr bool TC = sizeof(T) == 4;
+  cplx<T> twc[TC ? tw_cache_size(N, E) : 1];
+  if constexpr (TC) load_tw_cache<T, N, E>(twc, jl, stw);
   cplx<T> w[E], acc[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -732,7 +737,7 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_rpie
     // The transform's barriers also order the previous slot's term writes before the reads
     // below, and this slot's reads of buffer (b − 1) before the writes of slot b + 1.
     const int lb = FITS ? S::base_row(line) : line * PLD;
-    line_fft<T, N, E, true, At, true>(v, jl, lre + lb, lim + lb, stw, twc);
+    line_fft<T, N, E, true, At, TC>(v, jl, lre + lb, lim + lb, stw, twc);
     if (upd_obj && b > b0) {
       store_sum(b - 1, DB ? (b - 1) & 1 : 0);
       if constexpr (!DB) __syncthreads();
@@ -790,8 +795,9 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_sum(
   constexpr int LDW = FITS ? S::LDS_WORDS : M * G * PLD;
   __shared__ T lre[LDW], lim[LDW];
   __shared__ cplx<T> stw[N];
-  constexpr bool DB = 2 * LDW * sizeof(T) + N * sizeof(cplx<T>) + 2 * TW * sizeof(cplx<T>) <=
-                      160 * 1024;
+  constexpr bool DB = sizeof(T) == 4 && 2 * LDW * sizeof(T) + N * sizeof(cplx<T>) +
+                                                2 * TW * sizeof(cplx<T>) <=
+                                            160 * 1024;
   constexpr int NBUF = DB ? 2 : 1;
   __shared__ cplx<T> terms[NBUF * TW];
   const int tid = threadIdx.x;
