@@ -350,7 +350,6 @@ class Engine : public EngineBase {
   using S = RowShape<T, N>;    // pass A
   using SR = RowShapeC<T, N>;  // pass C
   using SC = ColShape<T, N>;   // column passes
-  using SB = BShape<T, N>;     // pass B
   static constexpr int n = N * N;
 
  public:
@@ -2919,7 +2918,7 @@ class Engine : public EngineBase {
     afar_tmp_.ensure(sizeof(T) * cap);
     prev_.ensure(sizeof(T) * 2);
     icalc_.ensure(sizeof(T) * cap * n);
-    xi_part_.ensure(sizeof(double) * 2 * cap * SB::NBLK);
+    xi_part_.ensure(sizeof(double) * 2 * cap * b_blocks());
     xi_part2_.ensure(sizeof(double) * 2 * cap * aux_blocks());
     dots_part_.ensure(sizeof(double) * 6 * cap * aux_blocks());
     sums_.ensure(sizeof(double) * 6 * cap);
@@ -3622,7 +3621,7 @@ class Engine : public EngineBase {
         pass_b<B_ICALC>(ord, nb, ba);
       run(K_OTHER, [&] {
         hipLaunchKernelGGL(k_lsqml_xi<T>, dim3(1), dim3(THREADS), 0, stream_,
-                           xi_part_.as<double>(), int(SB::NBLK), nb, prev_.as<T>(),
+                           xi_part_.as<double>(), b_blocks(), nb, prev_.as<T>(),
                            afar_tmp_.as<T>(), prev_.as<T>() + 1);
         hipLaunchKernelGGL(k_lsqml_xi_sums<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
                            icalc_.as<T>(), counts_.as<float>(), ord, n, prev_.as<T>() + 1,
@@ -3845,7 +3844,7 @@ class Engine : public EngineBase {
       pass_b<B_ICALC>(ord, nb, ba);
       run(K_OTHER, [&] {
         hipLaunchKernelGGL(k_lsqml_xi<T>, dim3(1), dim3(THREADS), 0, stream_,
-                           xi_part_.as<double>(), int(SB::NBLK), nb, prev_.as<T>(),
+                           xi_part_.as<double>(), b_blocks(), nb, prev_.as<T>(),
                            afar_tmp_.as<T>(), prev_.as<T>() + 1);
         hipLaunchKernelGGL(k_lsqml_xi_sums<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
                            icalc_.as<T>(), counts_.as<float>(), ord, n, prev_.as<T>() + 1,
@@ -4156,6 +4155,10 @@ class Engine : public EngineBase {
     });
   }
 
+  // Pass B's workgroups per frame.
+  int b_blocks() const {
+    return M_ <= kBWideModes ? BShape<T, N, 1>::NBLK : BShape<T, N, kMaxModes>::NBLK;
+  }
   int ntiles() const { return ntx_ * nty_; }
   // The tile kernels' split (SP of them share a tile's views; kernels.hpp): by the tile count.
   template <typename F>
@@ -4279,7 +4282,7 @@ class Engine : public EngineBase {
   // Scratch layout of llk_noalloc: the per-workgroup sums (4 doubles per frame and pass-B
   // workgroup), the 4 result sums, then the stack, each part 256-byte aligned.
   static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
-  size_t llk_part_bytes() const { return align256(sizeof(double) * 4 * nframe_ * SB::NBLK); }
+  size_t llk_part_bytes() const { return align256(sizeof(double) * 4 * nframe_ * b_blocks()); }
   size_t llk_scratch_bytes(size_t frames) const override {
     return llk_part_bytes() + 256 + sizeof(cplx<T>) * frames * M_ * n;
   }
@@ -4340,7 +4343,7 @@ class Engine : public EngineBase {
     pmax_.ensure(sizeof(T) * 1);
     order_.ensure(sizeof(int) * std::max<size_t>(1, nepoch * nframe_));
     eord_.ensure(sizeof(int) * std::max<size_t>(1, nframe_));
-    llk_part_.ensure(sizeof(double) * 4 * nframe_ * SB::NBLK);
+    llk_part_.ensure(sizeof(double) * 4 * nframe_ * b_blocks());
     cap_ = std::max(cap_, cap);
     if (nslice_ > 1) inc_.ensure(sizeof(cplx<T>) * inc_slots() * cap_ * M_ * n);
     ensure_positions(cap_);
@@ -4404,7 +4407,7 @@ class Engine : public EngineBase {
         constexpr int MM = decltype(mm)::value;
         auto col = k_pass_b<T, N, MM, MODE, false>;
         auto row = k_pass_b<T, N, MM, MODE, true>;
-        hipLaunchKernelGGL(angular_ ? row : col, dim3(SB::NBLK, nb),
+        hipLaunchKernelGGL(angular_ ? row : col, dim3(b_blocks(), nb),
                            dim3(pass_b_threads<T, N, MM>()), 0, stream_, stack(),
                            counts_.as<float>(), ord, llk_parts(), tw_.as<cplx<T>>(),
                            ba, norm);
@@ -4447,7 +4450,7 @@ class Engine : public EngineBase {
     }
     run(K_LLK, [&] {
       hipLaunchKernelGGL(k_llk_reduce, dim3(1), dim3(THREADS), 0, stream_, llk_parts(),
-                         int(nframe_ * SB::NBLK), result);
+                         int(nframe_ * b_blocks()), result);
     });
   }
 
@@ -4676,7 +4679,7 @@ class Engine : public EngineBase {
       pass_b<B_ICALC>(ord, nb, ba);
       run(K_OTHER, [&] {
         hipLaunchKernelGGL(k_lsqml_xi<T>, dim3(1), dim3(THREADS), 0, stream_,
-                           xi_part_.as<double>(), int(SB::NBLK), nb, prev_.as<T>(),
+                           xi_part_.as<double>(), b_blocks(), nb, prev_.as<T>(),
                            afar_tmp_.as<T>(), prev_.as<T>() + 1);
         hipLaunchKernelGGL(k_lsqml_xi_sums<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
                            icalc_.as<T>(), counts_.as<float>(), ord, n, prev_.as<T>() + 1,

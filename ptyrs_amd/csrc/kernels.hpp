@@ -302,15 +302,26 @@ struct BArgs {
 // Pass B's lines: per mode, a stripe of CG columns (or rows) of N values, E per thread (16
 // float / 8 double: one LDS exchange fewer than the column passes' 8 / 4). Every mode of the
 // stripe has its own group of threads and its own exchange region.
+// At 512: double up to kBWideModes modes keeps the 64-byte stripe (more modes' regions of LDS
+// would leave one workgroup on a CU), 315 µs against 425 on half of it (2 modes, 75 slots). Float
+// takes half of it, and up to four modes 8 values per thread: 16 exchange no less at 512 (16·16·2
+// against 8·8·8) but hold 178 registers, two waves per SIMD (2 modes, 100 slots: 342 µs, so 281;
+// on the whole stripe 321; 4 modes 781, so 691).
+constexpr int kBWideModes = 2;
 template <typename T>
-constexpr int pass_b_lines(int n) {
-  return (sizeof(T) == 4 ? 8 : 4) / (n >= 512 ? 2 : 1);
+constexpr int pass_b_lines(int n, int m) {
+  if (sizeof(T) == 4) return n >= 512 ? 4 : 8;
+  return n >= 512 && m > kBWideModes ? 2 : 4;
 }
-template <typename T, int N>
-using BShape = Lines<N, choose_e(N, sizeof(T) == 4 ? 16 : 8), 1024, pass_b_lines<T>(N), sizeof(T)>;
+template <typename T>
+constexpr int pass_b_e(int n, int m) {
+  return choose_e(n, sizeof(T) == 8 || (n >= 512 && m <= 4) ? 8 : 16);
+}
+template <typename T, int N, int M>
+using BShape = Lines<N, pass_b_e<T>(N, M), 1024, pass_b_lines<T>(N, M), sizeof(T)>;
 template <typename T, int N, int M>
 constexpr int pass_b_threads() {
-  return M * BShape<T, N>::NT;
+  return M * BShape<T, N, M>::NT;
 }
 
 // Grid (NBLK, nb) of BShape. Mode group m of each workgroup transforms mode m of the stripe;
@@ -337,7 +348,7 @@ template <typename T, int N, int M, int MODE, bool ROW>
 __global__ __launch_bounds__((pass_b_threads<T, N, M>())) void k_pass_b(
     cplx<T>* __restrict__ psi, const float* __restrict__ counts, const int* __restrict__ order,
     double* __restrict__ llk_part, const cplx<T>* __restrict__ tw, BArgs<T> ba, T norm) {
-  using S = BShape<T, N>;
+  using S = BShape<T, N, M>;
   constexpr int E = S::E, TL = S::TL, CG = S::L;
   constexpr int NT = pass_b_threads<T, N, M>();
   // Each group's region holds its exchanges and, after the forward transform, its intensities.
@@ -378,8 +389,9 @@ __global__ __launch_bounds__((pass_b_threads<T, N, M>())) void k_pass_b(
   for (int e = 0; e < E; ++e) v[e] = bld<T>(plane, i0 * cb, e * step * cb);
   stage_twiddles<T, N, NT>(stw, tw);
   // The forward and inverse transforms share the lane's twiddles, held in registers for float
-  // (for double they would cost a wave per SIMD).
-  constexpr bool TC = sizeof(T) == 4;
+  // where they are few (for double, and for the 23 of 16 values per thread at 512, they would cost
+  // a wave per SIMD or more).
+  constexpr bool TC = sizeof(T) == 4 && tw_cache_size(N, E) <= 16;
   cplx<T> twc[TC ? tw_cache_size(N, E) : 1];
   if constexpr (TC) load_tw_cache<T, N, E>(twc, jl, stw);
   line_fft<T, N, E, false, At, TC>(v, jl, re, im, stw, twc);
