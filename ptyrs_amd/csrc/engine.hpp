@@ -4209,10 +4209,13 @@ class Engine : public EngineBase {
                  int* count, const T* W2, int M, int nyo, int nxo, T* D, T* tilemax,
                  const cplx<T>* Wv) {
     split_tiles([&](auto sp) {
-      constexpr int SP = decltype(sp)::value;
-      hipLaunchKernelGGL((k_bin_tiles<T, SP>), dim3(ntiles()), dim3(THREADS * SP), 0, stream_,
-                         corner, ord, nb, side, ntx, cap, list, count, W2, M, nyo, nxo, D,
-                         tilemax, Wv);
+      mode_chunk(false, [&](auto mm) {
+        constexpr int SP = decltype(sp)::value, VW = decltype(mm)::value;
+        if constexpr (VW > 0)
+          hipLaunchKernelGGL((k_bin_tiles<T, SP, VW>), dim3(ntiles()), dim3(THREADS * SP), 0,
+                             stream_, corner, ord, nb, side, ntx, cap, list, count, W2, M, nyo,
+                             nxo, D, tilemax, Wv);
+      });
     });
   }
   void obj_dir(cplx<T>* dO, const cplx<T>* Wt, const cplx<T>* chi, int side, int M,
@@ -4339,7 +4342,8 @@ class Engine : public EngineBase {
     lcount_.ensure(sizeof(int) * size_t(ntiles()));
     tilemax_.ensure(sizeof(T) * size_t(ntiles()));
     D_.ensure(sizeof(T) * size_t(M_) * nyo_ * nxo_);
-    W2_.ensure(sizeof(T) * size_t(M_) * n);
+    const int vw = overlap_modes(M_);
+    W2_.ensure(sizeof(T) * size_t((M_ + vw - 1) / vw * vw) * n);
     pmax_.ensure(sizeof(T) * 1);
     order_.ensure(sizeof(int) * std::max<size_t>(1, nepoch * nframe_));
     eord_.ensure(sizeof(int) * std::max<size_t>(1, nframe_));
@@ -4353,7 +4357,7 @@ class Engine : public EngineBase {
   void norm2_planes() {
     const int total = int(M_) * n;
     hipLaunchKernelGGL(k_norm2_planes<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
-                       (const cplx<T>*)Wt_.as<cplx<T>>(), W2_.as<T>(), total);
+                       (const cplx<T>*)Wt_.as<cplx<T>>(), W2_.as<T>(), n, overlap_modes(M_), total);
   }
 
   void probe_terms() {
@@ -4368,18 +4372,20 @@ class Engine : public EngineBase {
   // the probe terms Wt.
   template <bool H = false>
   // `obj`, `obj_nxo` and `corners` (nullable) replace the object plane, its width and the
-  // frames' corners (FullObject's tall windows).
+  // frames' corners (FullObject's tall windows); with `tilemax` the launch also takes the tiles'
+  // max into pmax_.
   void pass_a(const int* ord, int nb, bool omax,
               MixArgs<T, H> mix = MixArgs<T, H>{MIX_NONE, {}, {}, T(0), T(0)},
               const cplx<T>* waves = nullptr, const cplx<T>* obj = nullptr, int obj_nxo = 0,
-              const int2* corners = nullptr) {
+              const int2* corners = nullptr, const T* tilemax = nullptr) {
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(S::NBLK, nb * M_), dim3(S::NT), 0, stream_,
+      hipLaunchKernelGGL(kern, dim3(S::NBLK, nb * M_ + int(tilemax != nullptr)), dim3(S::NT), 0,
+                         stream_,
                          obj ? obj : O_.as<cplx<T>>(), obj ? obj_nxo : int(nxo_),
                          waves ? waves : Wt_.as<cplx<T>>(),
                          corners ? corners : corner_.as<int2>(), ord, M_, stack(),
                          omax ? omax_.as<T>() : nullptr, tw_.as<cplx<T>>(), mix,
-                         int(waves != nullptr));
+                         int(waves != nullptr), tilemax, ntiles(), pmax_.as<T>());
     };
     run(K_PASS_A, [&] {
       switch (mix.kind) {
@@ -4487,6 +4493,8 @@ class Engine : public EngineBase {
     }
     const bool upd_obj = p.has_obj_step != 0, upd_probe = p.has_probe_step != 0;
     const int nt = ntiles();
+    // Pass A's launch takes the tiles' max with it where its grid has room for the row.
+    const bool fold = upd_obj && size_t(nb) * M_ < 65535;
     if (upd_obj) {
       // W2_ holds |W_m|² of the batch-start probe terms (rpie_begin, then each batch's
       // k_rpie_updates; without probe updates the probe does not change).
@@ -4496,12 +4504,14 @@ class Engine : public EngineBase {
                            D_.as<T>(), tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
       });
-      run(K_OVERLAP, [&] {
-        hipLaunchKernelGGL(k_max_reduce<T>, dim3(1), dim3(MAX_THREADS), 0, stream_,
-                           tilemax_.as<T>(), nt, pmax_.as<T>());
-      });
+      if (!fold)
+        run(K_OVERLAP, [&] {
+          hipLaunchKernelGGL(k_max_reduce<T>, dim3(1), dim3(MAX_THREADS), 0, stream_,
+                             tilemax_.as<T>(), nt, pmax_.as<T>());
+        });
     }
-    pass_a(ord, nb, upd_probe);
+    pass_a(ord, nb, upd_probe, MixArgs<T>{MIX_NONE, {}, {}, T(0), T(0)}, nullptr, nullptr, 0,
+           nullptr, fold ? (const T*)tilemax_.as<T>() : nullptr);
     pass_b<B_RPIE>(ord, nb);
     const int chunk = chunk_of_m(nb);
     const int nchunk = (nb + chunk - 1) / chunk;

@@ -180,16 +180,26 @@ __global__ void k_zero(U* __restrict__ p, size_t count) {
     p[i] = U{};
 }
 
-// W2[i] = |Wt[i]|² over the M planes of the probe terms (the per-mode overlap's summands).
+// |W_m|² of the probe terms (the per-mode overlap's summands) as W2[group][pixel][vw], vw modes
+// of a pixel side by side (overlap_modes), so that the overlaps load a pixel's modes at once.
+__host__ __device__ constexpr int overlap_modes(int M) { return M == 1 ? 1 : M == 2 ? 2 : 4; }
+__device__ __forceinline__ size_t w2_at(int i, int n, int vw) {
+  const int m = i / n, j = i % n;
+  return ((size_t)(m / vw) * n + j) * vw + m % vw;
+}
 template <typename T>
-__global__ void k_norm2_planes(const cplx<T>* __restrict__ Wt, T* __restrict__ W2, int total) {
+__global__ void k_norm2_planes(const cplx<T>* __restrict__ Wt, T* __restrict__ W2, int n, int vw,
+                               int total) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < total) W2[i] = norm2(ld(Wt + i));
+  if (i < total) W2[w2_at(i, n, vw)] = norm2(ld(Wt + i));
 }
 
 // ---- pass A: gather O·P·q and transform rows ---------------------------------------------------
-// Grid (NBLK, nb·M). View (b, m) = (blockIdx.y / M, blockIdx.y % M). With `omax_part`, mode-0
-// workgroups also write max |O|² over their rows of the window.
+// Grid (NBLK, nb·M), with `tilemax` one row of workgroups more: the first of them takes the max
+// of the tiles' overlaps into pmax, which only pass C reads, so that it hides behind the
+// transforms (a launch of its own took 4.8 µs of a batch's 57 at 96² × 3 modes, 37 views). View
+// (b, m) = (y / M, y % M). With `omax_part`, mode-0 workgroups also write max |O|² over their rows
+// of the window.
 // The exit wave pass A transforms: PO itself, or DM's and RAAR's mix of PO with the waves
 // they carry across cycles (ptyrs/src/engine/ptycho.rs:643-731).
 enum Mix { MIX_NONE = 0, MIX_DM = 1, MIX_RAAR = 2, MIX_RAAR0 = 3 };
@@ -240,7 +250,8 @@ __global__ __launch_bounds__((RowShape<T, N>::NT)) void k_pass_a(
     const cplx<T>* __restrict__ O, int nxo, const cplx<T>* __restrict__ Wt,
     const int2* __restrict__ corner, const int* __restrict__ order, int M,
     cplx<T>* __restrict__ psi, T* __restrict__ omax_part, const cplx<T>* __restrict__ tw,
-    MixArgs<T, H> mix, int w_view) {
+    MixArgs<T, H> mix, int w_view, const T* __restrict__ tilemax, int ntile,
+    T* __restrict__ pmax) {
   using S = RowShape<T, N>;
   constexpr int E = S::E, TL = S::TL;
   __shared__ T lre[S::LDS_WORDS], lim[S::LDS_WORDS];
@@ -248,12 +259,21 @@ __global__ __launch_bounds__((RowShape<T, N>::NT)) void k_pass_a(
   __shared__ cplx<T> stw[N];
   const int tid = threadIdx.x, l = tid / TL, jl = tid % TL;
   const int y = blockIdx.x * S::L + l;
-  const int b = blockIdx.y / M, m = blockIdx.y % M;
+  const int view = int(blockIdx.y) - (tilemax != nullptr);
+  if (view < 0) {
+    if (blockIdx.x > 0) return;
+    T v = 0;
+    for (int i = tid; i < ntile; i += S::NT) v = tilemax[i] > v ? tilemax[i] : v;
+    v = block_reduce<S::NT>(v, red, MaxOp());
+    if (tid == 0) pmax[0] = v;
+    return;
+  }
+  const int b = view / M, m = view % M;
   stage_twiddles<T, N, S::NT>(stw, tw);
   const int f = order[b];
   const int2 c = corner[f];
   const cplx<T>* orow = O + (size_t)(c.x + y) * nxo + c.y;
-  const cplx<T>* wrow = Wt + ((size_t)(w_view ? int(blockIdx.y) : m) * N + y) * N;
+  const cplx<T>* wrow = Wt + ((size_t)(w_view ? view : m) * N + y) * N;
   const size_t crow = (((size_t)f * M + m) * N + y) * N;
   cplx<T> v[E];
   T mx = 0;
@@ -958,7 +978,7 @@ __device__ __forceinline__ void probe_apply_blk(int blk, cplx<T>* __restrict__ P
   st(P + i, p);
   const cplx<T> w = p * ld(q + i % n);
   st(Wt + i, w);
-  if (W2) W2[i] = norm2(w);
+  if (W2) W2[w2_at(i, n, overlap_modes(total / n))] = norm2(w);
 }
 
 template <typename T>
@@ -1018,18 +1038,23 @@ __device__ __forceinline__ void merge_groups(kahan<T>& sr, kahan<T>& si, T* part
 }
 
 // One workgroup per object tile: (1) the batch slots whose N×N window meets the tile, in slot
-// order, compacted with wave ballots into list[tile][·] and count[tile]; (2) with `W2` (|W_m|²
-// per mode, W = P·q) or `Wv` (every view's own wave W, plane slot·M + m, under position
+// order, compacted with wave ballots into list[tile][·] and count[tile]; (2) with `W2` (|W_m|²,
+// W = P·q, VW modes of a pixel side by side) or `Wv` (every view's own wave W, plane slot·M + m, under position
 // offsets), each pixel's batch overlap D_m = Σ_views |W_m|² per mode into D[m][pixel] and the
 // tile max of Σ_m D_m (rPIE's regulariser max).
-template <typename T, int SP>
+template <typename T, int VW>
+struct alignas(VW * sizeof(T)) ModeVec {
+  T v[VW];
+};
+
+template <typename T, int SP, int VW>
 __global__ __launch_bounds__(THREADS * SP) void k_bin_tiles(
     const int2* __restrict__ corner, const int* __restrict__ order, int nb, int N, int ntx,
     int cap, int* __restrict__ list, int* __restrict__ count, const T* __restrict__ W2,
     int M, int nyo, int nxo, T* __restrict__ D, T* __restrict__ tilemax,
     const cplx<T>* __restrict__ Wv) {
   constexpr int BT = THREADS * SP;
-  constexpr int MM = 4;  // modes per chunk of overlaps held in registers
+  constexpr int MM = VW;  // modes per chunk of overlaps held in registers
   __shared__ int wave_n[BT / 64];
   __shared__ int base_s;
   __shared__ T red[BT];
@@ -1093,25 +1118,30 @@ __global__ __launch_bounds__(THREADS * SP) void k_bin_tiles(
         __syncthreads();
       }
       if (X < nxo) {
-        // One slot at a time in this form is fastest (256² × 4 modes: 2 slots' loads together
-        // took 8 % longer, 4 slots 14 %, 8 slots 30 %, and a plain loop with the bounds test
-        // as a branch 31 %).
+        // One slot at a time in this form is fastest (256² × 4 modes with a load per mode: 2
+        // slots took 8 % longer, 4 slots 14 %, 8 slots 30 %, and a plain loop with the bounds
+        // test as a branch 31 %). A pixel's modes in one load: the overlaps of 100 views take
+        // 17.4 µs instead of 20.7, of all 1024 views 90 instead of 131.
         const int2 r = share_of<SP>(g, k);
+        const auto* planes =
+            reinterpret_cast<const ModeVec<T, VW>*>(W2) + (size_t)(m0 / VW) * n;
         for (int i = r.x; i < r.y; ++i) {
           const int x = X - cs[i].y, y = Y - cs[i].x;
           const bool ok = x >= 0 && x < N && y >= 0 && y < N;
-          T w2[MM];
+          ModeVec<T, VW> w2;
           if (ok) {
+            if (Wv) {
 #pragma unroll
-            for (int m = 0; m < MM; ++m)
-              if (m < mc)
-                w2[m] = Wv ? norm2(Wv[((size_t)bs[i] * M + m0 + m) * n + y * N + x])
-                           : W2[(size_t)(m0 + m) * n + y * N + x];
+              for (int m = 0; m < MM; ++m)
+                if (m < mc) w2.v[m] = norm2(Wv[((size_t)bs[i] * M + m0 + m) * n + y * N + x]);
+            } else {
+              w2 = planes[y * N + x];
+            }
           }
           if (ok) {
 #pragma unroll
             for (int m = 0; m < MM; ++m)
-              if (m < mc) dm[m] += w2[m];
+              if (m < mc) dm[m] += w2.v[m];
           }
         }
       }
