@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "download.hpp"
 #include "host.hpp"
 #include "kernels.hpp"
 #include "bh.hpp"
@@ -2889,7 +2890,12 @@ class Engine : public EngineBase {
     for (size_t i = 0; i < count; ++i) h[i] = cplx<T>{T(src[2 * i]), T(src[2 * i + 1])};
     PTYRS_HIP(hipMemcpy(d.p, h.data(), sizeof(cplx<T>) * count, hipMemcpyHostToDevice));
   }
+  DownloadRing ring_;
   void download_complex(const DevBuf& d, double* out, size_t count) {
+    if (ring_.takes(sizeof(cplx<T>) * count)) {
+      PTYRS_HIP(ring_.run(device_, stream_, d.as<const cplx<T>>(), count, out));
+      return;
+    }
     std::vector<cplx<T>> h(count);
     PTYRS_HIP(hipStreamSynchronize(stream_));
     PTYRS_HIP(hipMemcpy(h.data(), d.p, sizeof(cplx<T>) * count, hipMemcpyDeviceToHost));
