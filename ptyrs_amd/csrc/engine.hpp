@@ -1103,7 +1103,8 @@ class Engine : public EngineBase {
                            tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_,
                            g, tw_.as<cplx<T>>());
-        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                            gP_.as<cplx<T>>(), (const cplx<T>*)g,
                            (const double2*)offs_.as<double2>(), ord, nb, N, M_,
                            1.0 / double(n), int(s > 0));
@@ -1743,7 +1744,8 @@ class Engine : public EngineBase {
                                g, tw_.as<cplx<T>>());
             hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0,
                                stream_, g, tw_.as<cplx<T>>());
-            hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + 255) / 256, M_), dim3(256), 0,
+            hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0,
                                stream_, gP_.as<cplx<T>>(), (const cplx<T>*)g,
                                (const double2*)offs_.as<double2>(), ord, nb, N, M_,
                                1.0 / double(n), int(s > 0));
@@ -1948,7 +1950,8 @@ class Engine : public EngineBase {
         run(K_PASS_C, [&] { rows(true, K); });
         if (up)
           run(K_PROBE, [&] {
-            hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + 255) / 256, M_), dim3(256), 0,
+            hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0,
                                stream_, gP_.as<cplx<T>>(), (const cplx<T>*)win, N,
                                (const cplx<T>*)q_.as<cplx<T>>(), g, fo_tall_.as<int2>(), ord, nb,
                                N, M_, T(1), int(s > 0));
@@ -3045,7 +3048,8 @@ class Engine : public EngineBase {
       hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_, gg,
                          tw_.as<cplx<T>>());
       // g_P = conj(q)·Σ_b DFT⁻¹(G_b·exp(+2πi f·d_b))
-      hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+      hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                          bh_gP_.as<cplx<T>>(), (const cplx<T>*)gg, offs, ord, nb, N, M_,
                          1.0 / double(n), 0);
       inverse_planes(bh_gP_.as<cplx<T>>(), M_);
@@ -3185,7 +3189,8 @@ class Engine : public EngineBase {
       });
     }
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+      hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                          bh_gP_.as<cplx<T>>(),
                          fo ? (const cplx<T>*)fo_swin(0) : (const cplx<T>*)slice_obj(0),
                          fo ? N : int(nxo_), (const cplx<T>*)nullptr, (const cplx<T>*)chi,
@@ -3661,8 +3666,7 @@ class Engine : public EngineBase {
                          stream_, dPm_.as<cplx<T>>(), dP_.as<cplx<T>>(), nchunk, total, nb);
     });
     run(K_DOTS, [&] {
-      hipLaunchKernelGGL(k_lsqml_dots<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
-                         dO_.as<cplx<T>>(), O_.as<cplx<T>>(), int(nxo_), Wt_.as<cplx<T>>(),
+      lsqml_dots(xb, nb, dO_.as<cplx<T>>(), O_.as<cplx<T>>(), int(nxo_), Wt_.as<cplx<T>>(),
                          dPm_.as<cplx<T>>(), q_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
                          corner_.as<int2>(), ord, dots_part_.as<double>());
       hipLaunchKernelGGL(k_lsqml_step<T>, dim3(1), dim3(1024), 0, stream_,
@@ -3745,7 +3749,8 @@ class Engine : public EngineBase {
         });
       }
       run(K_PROBE, [&] {
-        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(), (const cplx<T>*)slice_obj(0), int(nxo_), q0,
                            (const cplx<T>*)chi, corner_.as<int2>(), ord, nb, N, M_, T(1), acc);
       });
@@ -3932,7 +3937,8 @@ class Engine : public EngineBase {
                            tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_, g,
                            tw_.as<cplx<T>>());
-        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(), (const cplx<T>*)g,
                            (const double2*)offs_.as<double2>(), ord, nb, N, M_,
                            1.0 / (double(n) * double(nb)));
@@ -3960,7 +3966,8 @@ class Engine : public EngineBase {
       });
     } else {
       run(K_PROBE, [&] {
-        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(),
                            fo ? (const cplx<T>*)fo_swin(0) : (const cplx<T>*)slice_obj(0),
                            fo ? N : int(nxo_), q0, (const cplx<T>*)chi,
@@ -3972,8 +3979,7 @@ class Engine : public EngineBase {
     const double lam = 1.2e-7 * scale_ * double(M_);
     run(K_OTHER, [&] {
       if (fo) fo_dir_windows(slice_dir(0), nb);
-      hipLaunchKernelGGL(k_lsqml_dots<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
-                         fo ? (const cplx<T>*)fo_dwin_.as<cplx<T>>()
+      lsqml_dots(xb, nb, fo ? (const cplx<T>*)fo_dwin_.as<cplx<T>>()
                             : (const cplx<T>*)slice_dir(0),
                          fo ? (const cplx<T>*)fo_swin(0) : (const cplx<T>*)slice_obj(0),
                          fo ? N : int(nxo_), wv.w0, (const cplx<T>*)dPm_.as<cplx<T>>(),
@@ -4236,6 +4242,17 @@ class Engine : public EngineBase {
                            stream_, dO, Wt, chi, side, M, corner, ord, list, count, cap, nyo,
                            nxo, ntx, pre, floor, per_view, q, q_frame, accumulate);
       });
+    });
+  }
+  void lsqml_dots(int xb, int nb, const cplx<T>* dO, const cplx<T>* O, int nxo,
+                  const cplx<T>* Wt, const cplx<T>* dP, const cplx<T>* q, const cplx<T>* chi,
+                  int side, int M, const int2* corner, const int* ord, double* part,
+                  int per_view = 0, const cplx<T>* qu = nullptr) {
+    mode_chunk(false, [&](auto mm) {
+      constexpr int MM = decltype(mm)::value;
+      if constexpr (MM > 0)
+        hipLaunchKernelGGL((k_lsqml_dots<T, MM>), dim3(xb, nb), dim3(THREADS), 0, stream_, dO, O,
+                           nxo, Wt, dP, q, chi, side, M, corner, ord, part, per_view, qu);
     });
   }
   template <bool H>
@@ -4638,7 +4655,8 @@ class Engine : public EngineBase {
                            tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_, g,
                            tw_.as<cplx<T>>());
-        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
+        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+                           dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(), (const cplx<T>*)g,
                            (const double2*)offs_.as<double2>(), ord, nb, N, M_,
                            1.0 / (double(n) * double(nb)));
@@ -4752,8 +4770,7 @@ class Engine : public EngineBase {
       // longer needed).
       fo_object_spectrum(dO_.as<cplx<T>>());
       fo_windows<AS_PLAIN>(fo_spec_.as<cplx<T>>(), nb, 0, fo_dwin_.p, (long long)n);
-      hipLaunchKernelGGL(k_lsqml_dots<T>, dim3(xb, nb), dim3(THREADS), 0, stream_,
-                         (const cplx<T>*)fo_dwin_.as<cplx<T>>(),
+      lsqml_dots(xb, nb, (const cplx<T>*)fo_dwin_.as<cplx<T>>(),
                          (const cplx<T>*)fo_win_.as<cplx<T>>(), N, W, dPm_.as<cplx<T>>(),
                          q_.as<cplx<T>>(), chi, N, M_, fo_tall_.as<int2>(), ord,
                          dots_part_.as<double>(), wview);

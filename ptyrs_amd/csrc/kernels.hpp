@@ -26,6 +26,8 @@
 namespace ptyrs {
 
 constexpr int THREADS = 256;
+// The slot and chunk sums over 64 pixels a workgroup: 16 groups of a wave each.
+constexpr int REDUCE_THREADS = 1024, REDUCE_PX = 64;
 
 // Elements per thread for a line of n: `pref` where its radix plan exists and the line fits in
 // THREADS_MAX threads, else the first divisor of n that has a plan.
@@ -914,6 +916,23 @@ __global__ __launch_bounds__((pass_c_sum_threads<T, N, M>())) void k_pass_c_sum(
   }
 }
 
+// The Kahan pairs of a workgroup's BT/px thread groups of px threads into group 0's, in group
+// order. `part` holds 4·BT values; all threads call it.
+template <typename T, int BT>
+__device__ __forceinline__ void merge_px(kahan<T>& sr, kahan<T>& si, int px, T* part) {
+  const int t = threadIdx.x;
+  part[t] = sr.s;
+  part[BT + t] = sr.c;
+  part[2 * BT + t] = si.s;
+  part[3 * BT + t] = si.c;
+  __syncthreads();
+  if (t < px)
+    for (int k = 1; k < BT / px; ++k) {
+      sr.merge(part[k * px + t], part[BT + k * px + t]);
+      si.merge(part[2 * BT + k * px + t], part[3 * BT + k * px + t]);
+    }
+}
+
 // Complex sums over `nchunk` planes of `total` values: a workgroup of BT threads takes PX
 // neighbouring elements, its BT/PX thread groups a contiguous share of the chunks each, and the
 // groups' Kahan pairs meet in LDS in group order. `part` holds 4·BT values. Returns true in the
@@ -940,19 +959,7 @@ __device__ __forceinline__ bool chunk_sum(const cplx<T>* __restrict__ src, int n
         }
     }
   }
-  if (ng > 1) {
-    const int t = threadIdx.x;
-    part[t] = sr.s;
-    part[BT + t] = sr.c;
-    part[2 * BT + t] = si.s;
-    part[3 * BT + t] = si.c;
-    __syncthreads();
-    if (g == 0)
-      for (int k = 1; k < ng; ++k) {
-        sr.merge(part[k * px + t], part[BT + k * px + t]);
-        si.merge(part[2 * BT + k * px + t], part[3 * BT + k * px + t]);
-      }
-  }
+  if (ng > 1) merge_px<T, BT>(sr, si, px, part);
   return g == 0 && i < total;
 }
 
@@ -1462,13 +1469,13 @@ __global__ __launch_bounds__(THREADS) void k_probe_mean(cplx<T>* __restrict__ dP
 // over modes and the workgroup's pixels, dop = dO_window·W·qu, dpo = O_window·dP_m·q, W = W_m or
 // with per_view the slot's own plane (a moved probe), qu nullable (1).
 // Grid (nblk, nb). ptyrs/src/engine/lsqml.rs:300-318
-template <typename T>
+template <typename T, int MM>
 __global__ __launch_bounds__(THREADS) void k_lsqml_dots(
     const cplx<T>* __restrict__ dO, const cplx<T>* __restrict__ O, int nxo,
     const cplx<T>* __restrict__ Wt, const cplx<T>* __restrict__ dP, const cplx<T>* __restrict__ q,
     const cplx<T>* __restrict__ chi, int N, int M, const int2* __restrict__ corner,
-    const int* __restrict__ order, double* __restrict__ part, int per_view = 0,
-    const cplx<T>* __restrict__ qu = nullptr) {
+    const int* __restrict__ order, double* __restrict__ part, int per_view,
+    const cplx<T>* __restrict__ qu) {
   __shared__ double red[THREADS];
   const int b = blockIdx.y;
   const int2 c = corner[order[b]];
@@ -1481,17 +1488,29 @@ __global__ __launch_bounds__(THREADS) void k_lsqml_dots(
     cplx<T> dow = ld(dO + p);
     if (qu) dow = dow * ld(qu + j);
     const cplx<T>* wv = per_view ? Wt + (size_t)b * M * n : Wt;
-    for (int m = 0; m < M; ++m) {
-      const cplx<T> u = dow * ld(wv + (size_t)m * n + j);
-      const cplx<T> v = ow * ld(dP + (size_t)m * n + j) * qj;
-      const cplx<T> ch = ld(chi + ((size_t)b * M + m) * n + j);
-      const cplx<T> a12 = cmulc(v, u);  // u·conj(v)
-      s[0] += double(norm2(u));
-      s[1] += double(norm2(v));
-      s[2] += double(a12.x);
-      s[3] += double(a12.y);
-      s[4] += double(cmulc(u, ch).x);
-      s[5] += double(cmulc(v, ch).x);
+    for (int m0 = 0; m0 < M; m0 += MM) {
+      // MM modes' loads together: one mode at a time the field's loads were a chain of latencies.
+      cplx<T> w[MM], p[MM], ch[MM];
+#pragma unroll
+      for (int m = 0; m < MM; ++m)
+        if (m0 + m < M) {
+          w[m] = ld(wv + (size_t)(m0 + m) * n + j);
+          p[m] = ld(dP + (size_t)(m0 + m) * n + j);
+          ch[m] = ld(chi + ((size_t)b * M + m0 + m) * n + j);
+        }
+#pragma unroll
+      for (int m = 0; m < MM; ++m)
+        if (m0 + m < M) {
+          const cplx<T> u = dow * w[m];
+          const cplx<T> v = ow * p[m] * qj;
+          const cplx<T> a12 = cmulc(v, u);  // u·conj(v)
+          s[0] += double(norm2(u));
+          s[1] += double(norm2(v));
+          s[2] += double(a12.x);
+          s[3] += double(a12.y);
+          s[4] += double(cmulc(u, ch[m]).x);
+          s[5] += double(cmulc(v, ch[m]).x);
+        }
     }
   }
   for (int i = 0; i < 6; ++i) {
@@ -1859,27 +1878,43 @@ __global__ __launch_bounds__((RowShape<T, N>::NT)) void k_rows_ms(
   for (int e = 0; e < E; ++e) st(row + jl + TL * e, v[e]);
 }
 
-// The probe direction of slice 0: dP_m = scale·Σ_b conj(O_0[win_b]·q)·χ_0[b·M + m], summed in
-// slot order (Kahan); scale 1/nb for LSQML's frame mean, 1 for a gradient's sum, which
-// `accumulate` adds to dP. Grid (ceil(n/256), M). ptyrs/src/engine/lsqml.rs:200-229
+// Sums over a batch's slots per pixel and mode: REDUCE_PX pixels a workgroup of REDUCE_THREADS, 16
+// thread groups taking a contiguous share of the slots each. One thread per pixel left most of the
+// chip idle behind a chain over the slots (128 slots of 128² × 2 modes: 39 µs, 10.6 so; a 50-slot mean of moved spectra 30 µs, 11.6).
+__device__ __forceinline__ int2 slot_share(int g, int nb) {
+  constexpr int NG = REDUCE_THREADS / REDUCE_PX;
+  const int per = (nb + NG - 1) / NG;
+  const int lo = g * per, hi = lo + per;
+  return int2{lo < nb ? lo : nb, hi < nb ? hi : nb};
+}
+
+// The probe direction of slice 0: dP_m = scale·Σ_b conj(O_0[win_b]·q)·χ_0[b·M + m] (Kahan);
+// scale 1/nb for LSQML's frame mean, 1 for a gradient's sum, which `accumulate` adds to dP. Grid
+// (ceil(n/REDUCE_PX), M). ptyrs/src/engine/lsqml.rs:200-229
 template <typename T>
-__global__ void k_ms_probe_dir(cplx<T>* __restrict__ dP, const cplx<T>* __restrict__ O, int nxo,
-                               const cplx<T>* __restrict__ q, const cplx<T>* __restrict__ chi,
-                               const int2* __restrict__ corner, const int* __restrict__ order,
-                               int nb, int N, int M, T scale, int accumulate) {
+__global__ __launch_bounds__(REDUCE_THREADS) void k_ms_probe_dir(
+    cplx<T>* __restrict__ dP, const cplx<T>* __restrict__ O, int nxo,
+    const cplx<T>* __restrict__ q, const cplx<T>* __restrict__ chi,
+    const int2* __restrict__ corner, const int* __restrict__ order, int nb, int N, int M, T scale,
+    int accumulate) {
+  __shared__ T part[4 * REDUCE_THREADS];
   const int n = N * N;
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
+  const int j = blockIdx.x * REDUCE_PX + threadIdx.x % REDUCE_PX;
   const int m = blockIdx.y, y = j / N, x = j % N;
-  const cplx<T> qj = q ? ld(q + j) : cplx<T>{T(1), T(0)};
+  const int2 sh = slot_share(threadIdx.x / REDUCE_PX, nb);
   kahan<T> sr, si;
-  for (int b = 0; b < nb; ++b) {
-    const int2 c = corner[order[b]];
-    const cplx<T> o = ld(O + (size_t)(c.x + y) * nxo + c.y + x) * qj;
-    const cplx<T> g = cmulc(o, ld(chi + ((size_t)b * M + m) * n + j));
-    sr.add(g.x);
-    si.add(g.y);
+  if (j < n) {
+    const cplx<T> qj = q ? ld(q + j) : cplx<T>{T(1), T(0)};
+    for (int b = sh.x; b < sh.y; ++b) {
+      const int2 c = corner[order[b]];
+      const cplx<T> o = ld(O + (size_t)(c.x + y) * nxo + c.y + x) * qj;
+      const cplx<T> g = cmulc(o, ld(chi + ((size_t)b * M + m) * n + j));
+      sr.add(g.x);
+      si.add(g.y);
+    }
   }
+  merge_px<T, REDUCE_THREADS>(sr, si, REDUCE_PX, part);
+  if (threadIdx.x >= REDUCE_PX || j >= n) return;
   cplx<T> v = cplx<T>{sr.s, si.s} * scale;
   if (accumulate) v = v + ld(dP + (size_t)m * n + j);
   st(dP + (size_t)m * n + j, v);
@@ -2000,27 +2035,33 @@ __global__ void k_ramp_planes(cplx<T>* out, const cplx<T>* spec, const double2* 
              T((double(v.x) * s + double(v.y) * c) * scale)});
 }
 
-// The frame mean of spectra moved back: out[m] = scale·Σ_b G[b·M + m]·exp(+2πi f·d_b), slots in
-// order (Kahan). Grid (ceil(n/256), M). ptyrs/src/engine/lsqml.rs:207-229
+// The frame mean of spectra moved back: out[m] = scale·Σ_b G[b·M + m]·exp(+2πi f·d_b) (Kahan, the
+// slots shared out as in k_ms_probe_dir). Grid (ceil(n/REDUCE_PX), M).
+// ptyrs/src/engine/lsqml.rs:207-229
 // With `accumulate` the result is added to out (a sum over stacks, in stack order).
 template <typename T>
-__global__ void k_unramp_mean(cplx<T>* __restrict__ out, const cplx<T>* __restrict__ G,
-                              const double2* __restrict__ offs, const int* __restrict__ order,
-                              int nb, int N, int M, double scale, int accumulate = 0) {
+__global__ __launch_bounds__(REDUCE_THREADS) void k_unramp_mean(
+    cplx<T>* __restrict__ out, const cplx<T>* __restrict__ G, const double2* __restrict__ offs,
+    const int* __restrict__ order, int nb, int N, int M, double scale, int accumulate = 0) {
+  __shared__ T part[4 * REDUCE_THREADS];
   const int n = N * N;
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
+  const int j = blockIdx.x * REDUCE_PX + threadIdx.x % REDUCE_PX;
   const int m = blockIdx.y;
-  const double fy = dft_freq(j / N, N), fx = dft_freq(j % N, N);
+  const int2 sh = slot_share(threadIdx.x / REDUCE_PX, nb);
   kahan<T> sr, si;
-  for (int b = 0; b < nb; ++b) {
-    const double2 d = offs[order[b]];
-    double s, c;
-    sincos(2.0 * M_PI * (fy * d.x + fx * d.y), &s, &c);
-    const cplx<T> v = ld(G + ((size_t)b * M + m) * n + j);
-    sr.add(T(double(v.x) * c - double(v.y) * s));
-    si.add(T(double(v.x) * s + double(v.y) * c));
+  if (j < n) {
+    const double fy = dft_freq(j / N, N), fx = dft_freq(j % N, N);
+    for (int b = sh.x; b < sh.y; ++b) {
+      const double2 d = offs[order[b]];
+      double s, c;
+      sincos(2.0 * M_PI * (fy * d.x + fx * d.y), &s, &c);
+      const cplx<T> v = ld(G + ((size_t)b * M + m) * n + j);
+      sr.add(T(double(v.x) * c - double(v.y) * s));
+      si.add(T(double(v.x) * s + double(v.y) * c));
+    }
   }
+  merge_px<T, REDUCE_THREADS>(sr, si, REDUCE_PX, part);
+  if (threadIdx.x >= REDUCE_PX || j >= n) return;
   cplx<T> r{T(double(sr.s) * scale), T(double(si.s) * scale)};
   if (accumulate) r = r + ld(out + (size_t)m * n + j);
   st(out + (size_t)m * n + j, r);
@@ -2402,7 +2443,6 @@ __global__ __launch_bounds__(THREADS) void k_probe_sums(
 // pixels of one mode's num (or, y = M, of den), the chunks shared out over 16 thread groups.
 // One thread per pixel walking every chunk of every mode left 3/4 of the CUs idle at 128² and
 // took 252 µs for 256 chunks of 2 modes; this takes 21.
-constexpr int REDUCE_THREADS = 1024, REDUCE_PX = 64;
 template <typename T>
 __global__ __launch_bounds__(REDUCE_THREADS) void k_probe_reduce(
     const cplx<T>* __restrict__ num_part, const T* __restrict__ den_part, int nchunk, int n, int M,
