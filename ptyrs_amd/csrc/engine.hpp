@@ -881,10 +881,10 @@ class Engine : public EngineBase {
         const int nck = (nb + ck - 1) / ck;
         const bool dm = p.algorithm == PTYRS_DM && !first;
         run(K_PASS_C, [&] {
-          hipLaunchKernelGGL((k_pass_c_proj<T, N, H>), dim3(SR::NBLK, M_, nck), dim3(SR::NT), 0,
+          hipLaunchKernelGGL((k_pass_c_proj<T, N, H, false>), dim3(SR::NBLK, M_, nck), dim3(SR::NT), 0,
                              stream_, psi_.as<cplx<T>>(), cw, O_.as<cplx<T>>(), int(nxo_),
                              Wt_.as<cplx<T>>(), q_.as<cplx<T>>(), corner_.as<int2>(), ord, nb,
-                             M_, ck, int(dm), T(2.0 - p.mix), T(1.0 - p.mix), 0,
+                             M_, ck, int(dm), T(2.0 - p.mix), T(1.0 - p.mix),
                              (cplx<T>*)nullptr, (T*)nullptr, tw_.as<cplx<T>>());
         });
       }
@@ -984,11 +984,11 @@ class Engine : public EngineBase {
         const int ck = chunk_of(nb);
         const int nck = (nb + ck - 1) / ck;
         run(K_PASS_C, [&] {
-          hipLaunchKernelGGL((k_pass_c_proj<T, N, false>), dim3(SR::NBLK, M_, nck), dim3(SR::NT),
+          hipLaunchKernelGGL((k_pass_c_proj<T, N, false, false>), dim3(SR::NBLK, M_, nck), dim3(SR::NT),
                              0, stream_, psi_.as<cplx<T>>(), Carried<T, false>{carried},
                              O_.as<cplx<T>>(), int(nxo_), ws, q_.as<cplx<T>>(),
                              corner_.as<int2>(), ord, nb, M_, ck, int(dm), T(2.0 - p.mix),
-                             T(1.0 - p.mix), 0, (cplx<T>*)nullptr, (T*)nullptr,
+                             T(1.0 - p.mix), (cplx<T>*)nullptr, (T*)nullptr,
                              tw_.as<cplx<T>>(), 1);
         });
         if (pos_refine_) {
@@ -1229,11 +1229,11 @@ class Engine : public EngineBase {
         const int ck = chunk_of(nb);
         const int nck = (nb + ck - 1) / ck;
         run(K_PASS_C, [&] {
-          hipLaunchKernelGGL((k_pass_c_proj<T, N, false>), dim3(SR::NBLK, M_, nck), dim3(SR::NT),
+          hipLaunchKernelGGL((k_pass_c_proj<T, N, false, false>), dim3(SR::NBLK, M_, nck), dim3(SR::NT),
                              0, stream_, psi_.as<cplx<T>>(), Carried<T, false>{carried},
                              (const cplx<T>*)win, N, Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
                              fo_tall_.as<int2>(), ord, nb, M_, ck, int(dm), T(2.0 - p.mix),
-                             T(1.0 - p.mix), 0, (cplx<T>*)nullptr, (T*)nullptr,
+                             T(1.0 - p.mix), (cplx<T>*)nullptr, (T*)nullptr,
                              tw_.as<cplx<T>>(), 0);
         });
         if (pos_refine_) {
@@ -1729,12 +1729,13 @@ class Engine : public EngineBase {
         pass_b<B_GRAD>(ord, nb);
         // One slot per chunk: each frame's conj(q·O)·g of its own.
         run(K_PASS_C, [&] {
-          hipLaunchKernelGGL((k_pass_c_proj<T, N, false>), dim3(SR::NBLK, M_, nb),
+          const auto pass_c = up ? k_pass_c_proj<T, N, false, true> : k_pass_c_proj<T, N, false, false>;
+          hipLaunchKernelGGL(pass_c, dim3(SR::NBLK, M_, nb),
                              dim3(SR::NT), 0, stream_, psi_.as<cplx<T>>(),
                              Carried<T, false>{carried_.as<cplx<T>>()}, O_.as<cplx<T>>(),
                              int(nxo_), Wt_.as<cplx<T>>(), q_.as<cplx<T>>(),
-                             corner_.as<int2>(), ord, nb, M_, 1, 0, T(0), T(0), int(up), g,
-                             pden1_.as<T>(), tw_.as<cplx<T>>());
+                             corner_.as<int2>(), ord, nb, M_, 1, 0, T(0), T(0), g,
+                             pden1_.as<T>(), tw_.as<cplx<T>>(), 0);
         });
         if (up) {
           run(K_PROBE, [&] {

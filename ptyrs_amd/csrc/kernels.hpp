@@ -2340,15 +2340,16 @@ __global__ __launch_bounds__(1024) static void k_pos_step(const double* __restri
 // Pass C of the projection algorithms. Grid (NBLK, M, nchunk); each workgroup runs over the
 // slots of its chunk: inverse row transform of the projected field Π, then the new carried wave
 // ψ' = Π (AP, RAAR) or Π + (1 − a)·(PO − R) with R = (2 − a)·PO − (1 − a)·ψ (DM), written to
-// carried[frame]. With `probe_sums` (AP: both updates read the old arrays) it adds
-// conj(q·O)·ψ' and |O|² of the slot's window into per-chunk partials. With w_view every slot's
+// carried[frame]. With PS (ML under offsets) it adds conj(q·O)·ψ' and |O|² of the slot's window
+// into per-chunk partials; a runtime switch held their registers (157 at 512 in float) for the
+// projections too (512² × 2 modes, 100 slots of DM: 320 µs, 216 so). With w_view every slot's
 // mode has its own wave W (plane slot·M + m of Wt, a moved probe) in PO.
-template <typename T, int N, bool H = false>
+template <typename T, int N, bool H, bool PS>
 __global__ __launch_bounds__((RowShapeC<T, N>::NT)) void k_pass_c_proj(
     const cplx<T>* __restrict__ psi, Carried<T, H> carried, const cplx<T>* __restrict__ O,
     int nxo, const cplx<T>* __restrict__ Wt, const cplx<T>* __restrict__ q,
     const int2* __restrict__ corner, const int* __restrict__ order, int nb, int M, int chunk,
-    int dm, T c0, T c1, int probe_sums, cplx<T>* __restrict__ num_part, T* __restrict__ den_part,
+    int dm, T c0, T c1, cplx<T>* __restrict__ num_part, T* __restrict__ den_part,
     const cplx<T>* __restrict__ tw, int w_view = 0) {
   using S = RowShapeC<T, N>;
   constexpr int E = S::E, TL = S::TL;
@@ -2361,15 +2362,17 @@ __global__ __launch_bounds__((RowShapeC<T, N>::NT)) void k_pass_c_proj(
   const int b0 = ch * chunk;
   const int b1 = b0 + chunk < nb ? b0 + chunk : nb;
   stage_twiddles<T, N, S::NT>(stw, tw);
-  cplx<T> w[E], qq[E], acc[E];
-  T den[E];
+  cplx<T> w[E], qq[PS ? E : 1], acc[PS ? E : 1];
+  T den[PS ? E : 1];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int x = jl + TL * e;
     w[e] = ld(Wt + (size_t)m * n + (size_t)y * N + x);
-    qq[e] = ld(q + (size_t)y * N + x);
-    acc[e] = cplx<T>{0, 0};
-    den[e] = 0;
+    if constexpr (PS) {
+      qq[e] = ld(q + (size_t)y * N + x);
+      acc[e] = cplx<T>{0, 0};
+      den[e] = 0;
+    }
   }
   for (int b = b0; b < b1; ++b) {
     const int f = order[b];
@@ -2395,13 +2398,13 @@ __global__ __launch_bounds__((RowShapeC<T, N>::NT)) void k_pass_c_proj(
         p = p + (po - r) * c1;
       }
       carried.put(crow + x, p);
-      if (probe_sums) {
+      if constexpr (PS) {
         acc[e] = acc[e] + cmulc(o * qq[e], p);
         den[e] += norm2(o);
       }
     }
   }
-  if (probe_sums) {
+  if constexpr (PS) {
     const size_t base = ((size_t)ch * M + m) * n + (size_t)y * N;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
