@@ -14,6 +14,7 @@
 #include "download.hpp"
 #include "host.hpp"
 #include "kernels.hpp"
+#include "frame.hpp"
 #include "bh.hpp"
 #include "opr.hpp"
 #include "sampling.hpp"
@@ -505,6 +506,8 @@ class Engine : public EngineBase {
     const size_t cap = std::min(p.batch_size, nframe_);
     ensure_workspace(cap, nepoch);
     if (full_object()) fo_ensure(cap_);
+    if (!pos_on_ && !full_object() && frame_path())
+      dP_.ensure(sizeof(cplx<T>) * cap_ * M_ * n);  // a slot a chunk
     if (pos_on_ && !full_object()) {
       // Under offsets pass C leaves one probe direction per frame, moved back and averaged.
       dP_.ensure(sizeof(cplx<T>) * cap_ * M_ * n);
@@ -4506,6 +4509,23 @@ class Engine : public EngineBase {
   }
 
   // One rPIE batch (ptyrs/src/engine/ptycho.rs:900-1086) from the batch-start object and probe.
+  // Whether rPIE's batches run k_rpie_frame, a frame a workgroup (frame.hpp): one mode, and one
+  // DFT to the detector (the angular spectrum takes two).
+  bool frame_path() const { return whole_frame<T, N>() && M_ == 1 && !angular_; }
+  void rpie_frames(const ptyrs_rpie_params& p, const int* ord, int nb) {
+    if constexpr (whole_frame<T, N>()) {
+      run(K_PASS_C, [&] {
+        hipLaunchKernelGGL((k_rpie_frame<T, N>), dim3(nb), dim3(FrameShape<T, N>::NT), 0, stream_,
+                           psi_.as<cplx<T>>(), (const cplx<T>*)O_.as<cplx<T>>(), int(nxo_),
+                           (const cplx<T>*)Wt_.as<cplx<T>>(), (const cplx<T>*)q_.as<cplx<T>>(),
+                           corner_.as<int2>(), ord, counts_.as<float>(),
+                           (const T*)D_.as<T>(), (const T*)tilemax_.as<T>(), ntiles(),
+                           T(p.obj_alpha), T(p.probe_alpha), int(p.has_obj_step != 0),
+                           int(p.has_probe_step != 0), dP_.as<cplx<T>>(),
+                           (const cplx<T>*)tw_.as<cplx<T>>(), T(1) / T(n));
+      });
+    }
+  }
   void rpie_batch(const ptyrs_rpie_params& p, const int* ord, int nb) {
     if (full_object()) {
       rpie_batch_sampled(p, ord, nb);
@@ -4519,6 +4539,7 @@ class Engine : public EngineBase {
     const int nt = ntiles();
     // Pass A's launch takes the tiles' max with it where its grid has room for the row.
     const bool fold = upd_obj && size_t(nb) * M_ < 65535;
+    const bool frames = frame_path();
     if (upd_obj) {
       // W2_ holds |W_m|² of the batch-start probe terms (rpie_begin, then each batch's
       // k_rpie_updates; without probe updates the probe does not change).
@@ -4528,31 +4549,36 @@ class Engine : public EngineBase {
                            D_.as<T>(), tilemax_.as<T>(),
                            (const cplx<T>*)nullptr);
       });
-      if (!fold)
+      if (!fold && !frames)
         run(K_OVERLAP, [&] {
           hipLaunchKernelGGL(k_max_reduce<T>, dim3(1), dim3(MAX_THREADS), 0, stream_,
                              tilemax_.as<T>(), nt, pmax_.as<T>());
         });
     }
-    pass_a(ord, nb, upd_probe, MixArgs<T>{MIX_NONE, {}, {}, T(0), T(0)}, nullptr, nullptr, 0,
-           nullptr, fold ? (const T*)tilemax_.as<T>() : nullptr);
-    pass_b<B_RPIE>(ord, nb);
-    const int chunk = chunk_of_m(nb);
-    const int nchunk = (nb + chunk - 1) / chunk;
-    run(K_PASS_C, [&] {
-      auto launch = [&](auto mm) {
-        constexpr int MM = decltype(mm)::value;
-        constexpr int G = rows_per_group(N, SR::L, MM);
-        hipLaunchKernelGGL((k_pass_c_rpie_sum<T, N, MM>), dim3(N / G, nchunk),
-                           dim3(pass_c_sum_threads<T, N, MM>()), 0, stream_, psi_.as<cplx<T>>(), O_.as<cplx<T>>(), int(nxo_),
-                           Wt_.as<cplx<T>>(), q_.as<cplx<T>>(), corner_.as<int2>(), ord, nb,
-                           omax_.as<T>(), int(S::NBLK), chunk, T(p.probe_alpha),
-                           int(upd_probe), dP_.as<cplx<T>>(), tw_.as<cplx<T>>(), int(upd_obj),
-                           (const T*)D_.as<T>(), int(nyo_), (const T*)pmax_.as<T>(),
-                           T(p.obj_alpha), 0, (cplx<T>*)nullptr);
-      };
-      with_modes(launch);
-    });
+    int nchunk = nb;
+    if (frames) {
+      rpie_frames(p, ord, nb);
+    } else {
+      pass_a(ord, nb, upd_probe, MixArgs<T>{MIX_NONE, {}, {}, T(0), T(0)}, nullptr, nullptr, 0,
+             nullptr, fold ? (const T*)tilemax_.as<T>() : nullptr);
+      pass_b<B_RPIE>(ord, nb);
+      const int chunk = chunk_of_m(nb);
+      nchunk = (nb + chunk - 1) / chunk;
+      run(K_PASS_C, [&] {
+        auto launch = [&](auto mm) {
+          constexpr int MM = decltype(mm)::value;
+          constexpr int G = rows_per_group(N, SR::L, MM);
+          hipLaunchKernelGGL((k_pass_c_rpie_sum<T, N, MM>), dim3(N / G, nchunk),
+                             dim3(pass_c_sum_threads<T, N, MM>()), 0, stream_, psi_.as<cplx<T>>(), O_.as<cplx<T>>(), int(nxo_),
+                             Wt_.as<cplx<T>>(), q_.as<cplx<T>>(), corner_.as<int2>(), ord, nb,
+                             omax_.as<T>(), int(S::NBLK), chunk, T(p.probe_alpha),
+                             int(upd_probe), dP_.as<cplx<T>>(), tw_.as<cplx<T>>(), int(upd_obj),
+                             (const T*)D_.as<T>(), int(nyo_), (const T*)pmax_.as<T>(),
+                             T(p.obj_alpha), 0, (cplx<T>*)nullptr);
+        };
+        with_modes(launch);
+      });
+    }
     if (upd_obj && upd_probe) {
       const int total = int(nprobe_ * n);
       run(K_OBJ_UPDATE, [&] {
