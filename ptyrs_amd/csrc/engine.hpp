@@ -827,7 +827,7 @@ class Engine : public EngineBase {
     list_all_.ensure(sizeof(int) * size_t(nt) * nb_all);
     count_all_.ensure(sizeof(int) * size_t(nt));
     const int nstack = int((nb_all + stack - 1) / stack);
-    const int chunk = ap ? chunk_of_m(int(stack)) : chunk_of(int(stack));
+    const int chunk = ap ? chunk_of_sum(int(stack)) : chunk_of(int(stack));
     const int nchunk = int((stack + chunk - 1) / chunk);
     pnum_part_.ensure(sizeof(cplx<T>) * size_t(nstack) * nchunk * M_ * n);
     pden_part_.ensure(sizeof(T) * size_t(nstack) * nchunk * n);
@@ -876,7 +876,7 @@ class Engine : public EngineBase {
           pass_c_sum<false>(ord, nb, nullptr, ap_probe, csum_.as<cplx<T>>(), true,
                             pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
                             pden_part_.as<T>() + size_t(s) * nchunk * n);
-          const int ck = chunk_of_m(nb), nck = (nb + ck - 1) / ck;
+          const int ck = chunk_of_sum(nb), nck = (nb + ck - 1) / ck;
           if (ap_probe && nck < nchunk) zero_partials(s, nck, nchunk);
           continue;
         }
@@ -1464,7 +1464,7 @@ class Engine : public EngineBase {
     list_all_.ensure(sizeof(int) * size_t(nt) * nframe_);
     count_all_.ensure(sizeof(int) * size_t(nt));
     const int nstack = int((nframe_ + stack - 1) / stack);
-    const int chunk = chunk_of_m(int(stack));
+    const int chunk = chunk_of_sum(int(stack));
     const int nchunk = int((stack + chunk - 1) / chunk);
     pnum_part_.ensure(sizeof(cplx<T>) * size_t(nstack) * nchunk * M_ * n);
     pden_part_.ensure(sizeof(T) * size_t(nstack) * nchunk * n);
@@ -1517,7 +1517,7 @@ class Engine : public EngineBase {
         pass_c_sum<false>(ord, nb, nullptr, up, csum_.as<cplx<T>>(), true,
                           pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
                           pden_part_.as<T>() + size_t(s) * nchunk * n);
-        const int ck = chunk_of_m(nb), nck = (nb + ck - 1) / ck;
+        const int ck = chunk_of_sum(nb), nck = (nb + ck - 1) / ck;
         if (up && nck < nchunk) zero_partials(s, nck, nchunk);
       }
       if (uo) {
@@ -3654,7 +3654,7 @@ class Engine : public EngineBase {
     });
     pass_c_sum<true>(ord, nb, linear ? (const T*)afar_tmp_.as<T>() : nullptr, true,
                      csum_.as<cplx<T>>(), false, dP_.as<cplx<T>>(), nullptr);
-    const int chunk = chunk_of_m(nb);
+    const int chunk = chunk_of_sum(nb);
     const int nchunk = (nb + chunk - 1) / chunk;
     run(K_OBJ_DIR, [&] {
       obj_dir(dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
@@ -4198,11 +4198,11 @@ class Engine : public EngineBase {
       f(std::integral_constant<int, 4>{});
   }
   // Pass C with the modes' terms summed over `nb` slots into `sums` (plane order[b] with
-  // by_frame, else b), chunk_of_m(nb) slots a chunk.
+  // by_frame, else b), chunk_of_sum(nb) slots a chunk.
   template <bool CHI>
   void pass_c_sum(const int* ord, int nb, const T* a_far, bool probe_dir, cplx<T>* sums,
                   bool by_frame, cplx<T>* num_part, T* den_part) {
-    const int chunk = chunk_of_m(nb);
+    const int chunk = chunk_of_sum(nb);
     const int nchunk = (nb + chunk - 1) / chunk;
     run(K_PASS_C, [&] {
       with_modes([&](auto mm) {
@@ -4286,6 +4286,13 @@ class Engine : public EngineBase {
     int nchunk = std::max(1, std::min(nb, (pass_c_blocks_ + per - 1) / per));
     return (nb + nchunk - 1) / nchunk;
   }
+  // The same for k_pass_c_sum (LSQML, AP, ML): it follows chi_blocks, in the workgroups of three
+  // quarters of it (768 of the default 1024: one round of three per CU).
+  int chunk_of_sum(int nb) const {
+    const int per = N / rows_per_group(N, SR::L, int(M_)), blocks = std::max(1, chi_blocks_ / 4 * 3);
+    int nchunk = std::max(1, std::min(nb, (blocks + per - 1) / per));
+    return (nb + nchunk - 1) / nchunk;
+  }
   int pass_c_blocks_ = kPassCBlocks, chi_blocks_ = kChiBlocks;
   static constexpr int kChiBlocks = 1024;
   static constexpr int kMaxLaunchBlocks = 8192;
@@ -4359,7 +4366,8 @@ class Engine : public EngineBase {
                     " modes holds more than 65535 views");
     psi_.ensure(sizeof(cplx<T>) * cap * M_ * n);
     omax_.ensure(sizeof(T) * cap * S::NBLK);
-    // chunk_of and chunk_of_m never cut more chunks than this, whatever the batch length.
+    // chunk_of, chunk_of_m and chunk_of_sum never cut more chunks than this, whatever the batch
+    // length.
     const size_t per =
         std::min(size_t(SR::NBLK) * M_, size_t(N / rows_per_group(N, SR::L, int(M_))));
     const size_t nchunk =
