@@ -200,10 +200,10 @@ def lsqml_bytes(c, r):
     n = N * N
     return {
         "pass_a": n * c + M * n * c,
-        # icalc pass: Ψ and counts in, icalc out; Poisson pass: Ψ and counts in, Ψ out
-        "pass_b": 3 * M * n * c + 8 * n + n * r,
-        "pass_c": 2 * M * n * c + n * c,             # Ψ' and the O window in, χ out
-        "obj_dir": M * n * c,                        # χ of every view over the tile in
+        "pass_b": 2 * M * n * c + 4 * n + n * r,     # Ψ and counts in, Ψ and icalc out
+        # Ψ' and the O window in, χ and the mode-summed object term out
+        "pass_c": 2 * M * n * c + 2 * n * c,
+        "obj_dir": n * c,                            # the summed term of every view in
         "dots": M * n * c + 2 * n * c,               # χ, the O and dO windows in
     }
 
