@@ -23,9 +23,9 @@ class DownloadRing {
  public:
   static constexpr int kWorkers = 4;
   static constexpr size_t kPiece = 512 * 1024;
-  // A worker per 2 MB from kMin on: each thread's first runtime call takes about 0.1 ms, and the
-  // ring's pages 1.6 ms to pin once, which a download of 2.4 MB did not earn back (0.6 ms a pass
-  // slower with four workers). Below kMin the ring is used, on the calling thread, once it exists.
+  // A worker per 2 MB from kMin on: the threads cost more than a small download has to gain (2.4 MB
+  // with four of them: 0.6 ms a pass slower than the plain copy), and so does making the ring (0.3
+  // ms). Below kMin it is used, on the calling thread, once it exists.
   static constexpr size_t kMin = 4 << 20, kPerWorker = 2 << 20;
 
   bool takes(size_t bytes) const { return bytes >= kMin || (host_ && bytes >= 2 * kPiece); }

@@ -326,21 +326,18 @@ struct BArgs {
 // stripe has its own group of threads and its own exchange region.
 // At 512: double up to kBWideModes modes keeps the 64-byte stripe (more modes' regions of LDS
 // would leave one workgroup on a CU), 315 µs against 425 on half of it (2 modes, 75 slots). Float
-// takes half of it, and up to four modes 8 values per thread: 16 exchange no less at 512 (16·16·2
-// against 8·8·8) but hold 178 registers, two waves per SIMD (2 modes, 100 slots: 342 µs, so 281;
-// on the whole stripe 321; 4 modes 781, so 691).
+// takes half of it (2 modes, 100 slots: 279 µs, on the whole stripe 360). 8 values per thread
+// instead of 16 took float the same time for 2 modes and 697 µs instead of 761 for 4; its other
+// order of roundings was not shown to be as close to 64 bits, so the plan stays.
 constexpr int kBWideModes = 2;
 template <typename T>
 constexpr int pass_b_lines(int n, int m) {
   if (sizeof(T) == 4) return n >= 512 ? 4 : 8;
   return n >= 512 && m > kBWideModes ? 2 : 4;
 }
-template <typename T>
-constexpr int pass_b_e(int n, int m) {
-  return choose_e(n, sizeof(T) == 8 || (n >= 512 && m <= 4) ? 8 : 16);
-}
 template <typename T, int N, int M>
-using BShape = Lines<N, pass_b_e<T>(N, M), 1024, pass_b_lines<T>(N, M), sizeof(T)>;
+using BShape =
+    Lines<N, choose_e(N, sizeof(T) == 4 ? 16 : 8), 1024, pass_b_lines<T>(N, M), sizeof(T)>;
 template <typename T, int N, int M>
 constexpr int pass_b_threads() {
   return M * BShape<T, N, M>::NT;
