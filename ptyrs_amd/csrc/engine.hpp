@@ -873,10 +873,10 @@ class Engine : public EngineBase {
         pass_a(ord, nb, false, mix);
         pass_b<B_AMPLITUDE>(ord, nb);
         if (ap) {
-          pass_c_sum<false>(ord, nb, nullptr, ap_probe, csum_.as<cplx<T>>(), true,
+          const int ck = chunk_within(chunk_of_sum(nb), nb, nchunk), nck = (nb + ck - 1) / ck;
+          pass_c_sum<false>(ord, nb, ck, nullptr, ap_probe, csum_.as<cplx<T>>(), true,
                             pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
                             pden_part_.as<T>() + size_t(s) * nchunk * n);
-          const int ck = chunk_of_sum(nb), nck = (nb + ck - 1) / ck;
           if (ap_probe && nck < nchunk) zero_partials(s, nck, nchunk);
           continue;
         }
@@ -1514,10 +1514,10 @@ class Engine : public EngineBase {
         const int* ord = iota_.as<int>() + f0;
         pass_a(ord, nb, false);
         pass_b<B_GRAD>(ord, nb);
-        pass_c_sum<false>(ord, nb, nullptr, up, csum_.as<cplx<T>>(), true,
+        const int ck = chunk_within(chunk_of_sum(nb), nb, nchunk), nck = (nb + ck - 1) / ck;
+        pass_c_sum<false>(ord, nb, ck, nullptr, up, csum_.as<cplx<T>>(), true,
                           pnum_part_.as<cplx<T>>() + size_t(s) * nchunk * M_ * n,
                           pden_part_.as<T>() + size_t(s) * nchunk * n);
-        const int ck = chunk_of_sum(nb), nck = (nb + ck - 1) / ck;
         if (up && nck < nchunk) zero_partials(s, nck, nchunk);
       }
       if (uo) {
@@ -3652,10 +3652,10 @@ class Engine : public EngineBase {
                          afar_tmp_.as<T>(), ord, nb, afar_all_.as<T>(),
                          log_.as<double>() + 3 * size_t(off), int(gauss), 3);
     });
-    pass_c_sum<true>(ord, nb, linear ? (const T*)afar_tmp_.as<T>() : nullptr, true,
-                     csum_.as<cplx<T>>(), false, dP_.as<cplx<T>>(), nullptr);
     const int chunk = chunk_of_sum(nb);
     const int nchunk = (nb + chunk - 1) / chunk;
+    pass_c_sum<true>(ord, nb, chunk, linear ? (const T*)afar_tmp_.as<T>() : nullptr, true,
+                     csum_.as<cplx<T>>(), false, dP_.as<cplx<T>>(), nullptr);
     run(K_OBJ_DIR, [&] {
       obj_dir(dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
               corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_), int(nyo_),
@@ -4049,7 +4049,8 @@ class Engine : public EngineBase {
   // LLK records the device holds before the host drains them (GpuOptions::llk_slots).
   size_t hist_slots_ = 8;
 
-  // Chunks of a short last stack hold no partials: zero them so every stack's slab sums.
+  // The chunks past a short last stack's (it cuts nchunk at most, chunk_within) hold no partials:
+  // zero them so every stack's slab sums.
   void zero_partials(int s, int from, int nchunk) {
     const size_t cn = size_t(M_) * n;
     zero(pnum_part_.as<cplx<T>>() + (size_t(s) * nchunk + from) * cn, (nchunk - from) * cn);
@@ -4094,7 +4095,7 @@ class Engine : public EngineBase {
     for (int s = 0; s < nstack; ++s) {
       const int f0 = int(s * stack);
       const int nb = std::min<int>(int(stack), int(nframe_) - f0);
-      const int ck = chunk_of(nb);
+      const int ck = chunk_within(chunk_of(nb), nb, nchunk);
       const int nck = (nb + ck - 1) / ck;
       run(K_PROBE, [&] {
         hipLaunchKernelGGL((k_probe_sums<T, H>), dim3((n + THREADS - 1) / THREADS, M_, nck),
@@ -4198,11 +4199,10 @@ class Engine : public EngineBase {
       f(std::integral_constant<int, 4>{});
   }
   // Pass C with the modes' terms summed over `nb` slots into `sums` (plane order[b] with
-  // by_frame, else b), chunk_of_sum(nb) slots a chunk.
+  // by_frame, else b), `chunk` slots a chunk.
   template <bool CHI>
-  void pass_c_sum(const int* ord, int nb, const T* a_far, bool probe_dir, cplx<T>* sums,
-                  bool by_frame, cplx<T>* num_part, T* den_part) {
-    const int chunk = chunk_of_sum(nb);
+  void pass_c_sum(const int* ord, int nb, int chunk, const T* a_far, bool probe_dir,
+                  cplx<T>* sums, bool by_frame, cplx<T>* num_part, T* den_part) {
     const int nchunk = (nb + chunk - 1) / chunk;
     run(K_PASS_C, [&] {
       with_modes([&](auto mm) {
@@ -4276,22 +4276,16 @@ class Engine : public EngineBase {
 
   // Pass C chunking: enough workgroups to fill the chip, few partial probe sums.
   int chunk_of(int nb) const {
-    const int per = SR::NBLK * M_;
-    int nchunk = std::max(1, std::min(nb, (chi_blocks_ + per - 1) / per));
-    return (nb + nchunk - 1) / nchunk;
+    return chunk_len(nb, SR::NBLK * M_, chi_blocks_);
   }
   // The same for rPIE's mode-summing pass C, whose workgroups hold G rows of every mode.
   int chunk_of_m(int nb) const {
-    const int per = N / rows_per_group(N, SR::L, int(M_));
-    int nchunk = std::max(1, std::min(nb, (pass_c_blocks_ + per - 1) / per));
-    return (nb + nchunk - 1) / nchunk;
+    return chunk_len(nb, N / rows_per_group(N, SR::L, int(M_)), pass_c_blocks_);
   }
   // The same for k_pass_c_sum (LSQML, AP, ML): it follows chi_blocks, in the workgroups of three
   // quarters of it (768 of the default 1024: one round of three per CU).
   int chunk_of_sum(int nb) const {
-    const int per = N / rows_per_group(N, SR::L, int(M_)), blocks = std::max(1, chi_blocks_ / 4 * 3);
-    int nchunk = std::max(1, std::min(nb, (blocks + per - 1) / per));
-    return (nb + nchunk - 1) / nchunk;
+    return chunk_len(nb, N / rows_per_group(N, SR::L, int(M_)), std::max(1, chi_blocks_ / 4 * 3));
   }
   int pass_c_blocks_ = kPassCBlocks, chi_blocks_ = kChiBlocks;
   static constexpr int kChiBlocks = 1024;

@@ -2,6 +2,7 @@
 // exit-wave plane phase, the detector index map of the exit transform, and seeded batches.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdint>
@@ -77,6 +78,20 @@ inline size_t required_obj_axis(const double* v, size_t count, double p, size_t 
   for (size_t i = 0; i < count; ++i) ext = std::fmax(ext, std::fabs(std::ceil(v[i] / p)) + 1.0);
   const size_t len = size_t(2.0 * ext) + frame + margin;
   return (len + 3) / 4 * 4;
+}
+
+// Slots per chunk of a launch over nb slots whose grid has `per` workgroups a chunk, for about
+// `blocks` workgroups in all.
+inline int chunk_len(int nb, int per, int blocks) {
+  const int nchunk = std::max(1, std::min(nb, (blocks + per - 1) / per));
+  return (nb + nchunk - 1) / nchunk;
+}
+
+// `chunk`, or the shortest longer chunk of nb slots that cuts no more than nchunk chunks. A
+// stack's buffers of chunk partials hold the chunks of a full stack, and chunk_len's count does
+// not grow steadily with nb: 128 slots for 48 chunks at most make 43 of 3, 48 slots 48 of 1.
+inline int chunk_within(int chunk, int nb, int nchunk) {
+  return std::max(chunk, (nb + nchunk - 1) / nchunk);
 }
 
 // SplitMix64 output function and the per-epoch batches of ptyrs/src/engine/batch.rs:7-38:
