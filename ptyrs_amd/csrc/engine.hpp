@@ -2903,6 +2903,9 @@ class Engine : public EngineBase {
       PTYRS_HIP(ring_.run(device_, stream_, d.as<const cplx<T>>(), count, out));
       return;
     }
+    download_plain(d, out, count);
+  }
+  void download_plain(const DevBuf& d, double* out, size_t count) {
     std::vector<cplx<T>> h(count);
     PTYRS_HIP(hipStreamSynchronize(stream_));
     PTYRS_HIP(hipMemcpy(h.data(), d.p, sizeof(cplx<T>) * count, hipMemcpyDeviceToHost));
@@ -3759,8 +3762,11 @@ class Engine : public EngineBase {
                            (const cplx<T>*)chi, corner_.as<int2>(), ord, nb, N, M_, T(1), acc);
       });
     }
-    download_complex(dO_, og, S * no);
-    download_complex(dPm_, pg, nprobe_ * n);
+    // Not through the ring: its workers compete with the host threads that a torch program's own
+    // conversions around this call keep busy (a 10 MB object gradient: 1000 frames of 256², 9.9 ms
+    // a call with the ring and 8.2 without; three slices at 128², 12.7 and 9.1).
+    download_plain(dO_, og, S * no);
+    download_plain(dPm_, pg, nprobe_ * n);
     flush_timing();
     *value = cost == PTYRS_POISSON ? v[0] : v[2] / 4.0;
   }
