@@ -28,7 +28,15 @@ class DownloadRing {
   // ms). Below kMin it is used, on the calling thread, once it exists.
   static constexpr size_t kMin = 4 << 20, kPerWorker = 2 << 20;
 
-  bool takes(size_t bytes) const { return bytes >= kMin || (host_ && bytes >= 2 * kPiece); }
+  // Whether a download of `bytes` goes through the ring, which this makes if it is wanted and
+  // missing. Pinned memory or events that are refused leave the caller its plain copy.
+  bool ready(size_t bytes) {
+    if (host_) return bytes >= 2 * kPiece;
+    if (bytes < kMin) return false;
+    if (prepare() == hipSuccess) return true;
+    (void)hipGetLastError();  // the next launch's check must not report it
+    return false;
+  }
 
   DownloadRing() = default;
   DownloadRing(const DownloadRing&) = delete;
@@ -39,21 +47,10 @@ class DownloadRing {
     if (host_) (void)hipHostFree(host_);
   }
 
-  hipError_t prepare() {
-    if (host_) return hipSuccess;
-    for (auto& e : done_) {
-      if (e) continue;
-      const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
-      if (r != hipSuccess) return r;
-    }
-    return hipHostMalloc(&host_, size_t(kSlots) * kPiece, hipHostMallocDefault);
-  }
-
-  // `count` complex values at `src`, after what `stream` holds, into out[2·count].
+  // `count` complex values at `src`, after what `stream` holds, into out[2·count], once the ring
+  // is ready.
   template <typename T>
   hipError_t run(int device, hipStream_t stream, const cplx<T>* src, size_t count, double* out) {
-    const hipError_t ready = prepare();
-    if (ready != hipSuccess) return ready;
     const size_t per = kPiece / sizeof(cplx<T>);
     const size_t pieces = (count + per - 1) / per;
     const size_t bytes = sizeof(cplx<T>) * count;
@@ -115,6 +112,20 @@ class DownloadRing {
 
  private:
   static constexpr int kSlots = 2 * kWorkers;
+  hipError_t prepare() {
+    for (auto& e : done_) {
+      if (e) continue;
+      const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+      if (r != hipSuccess) {
+        e = nullptr;
+        return r;
+      }
+    }
+    const hipError_t r =
+        hipHostMalloc(&host_, size_t(kSlots) * kPiece, hipHostMallocDefault);
+    if (r != hipSuccess) host_ = nullptr;
+    return r;
+  }
   void* at(int slot) const { return static_cast<char*>(host_) + size_t(slot) * kPiece; }
   void* host_ = nullptr;
   hipEvent_t done_[kSlots] = {};

@@ -2899,7 +2899,7 @@ class Engine : public EngineBase {
   }
   DownloadRing ring_;
   void download_complex(const DevBuf& d, double* out, size_t count) {
-    if (ring_.takes(sizeof(cplx<T>) * count)) {
+    if (ring_.ready(sizeof(cplx<T>) * count)) {
       PTYRS_HIP(ring_.run(device_, stream_, d.as<const cplx<T>>(), count, out));
       return;
     }
