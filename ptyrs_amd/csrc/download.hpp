@@ -3,7 +3,7 @@
 // while it widens another into the caller's pages. A pageable copy of the whole array into a
 // fresh host vector and one loop over it took 1.9 ms for a 1136² complex64 object and four 256²
 // modes (the vector's and the caller's page faults, the staged copy and the loop one after the
-// other); this takes 0.5.
+// other); this takes 0.7 once the ring is there.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -24,15 +24,20 @@ class DownloadRing {
   static constexpr int kWorkers = 4;
   static constexpr size_t kPiece = 512 * 1024;
   // A worker per 2 MB from kMin on: the threads cost more than a small download has to gain (2.4 MB
-  // with four of them: 0.6 ms a pass slower than the plain copy), and so does making the ring (0.3
-  // ms). Below kMin it is used, on the calling thread, once it exists.
+  // with four of them: 0.6 ms a pass slower than the plain copy). Below kMin it is used, on the
+  // calling thread, once it exists.
   static constexpr size_t kMin = 4 << 20, kPerWorker = 2 << 20;
+  // Large downloads that go without: the ring's pinned memory takes 0.35 ms and its first use as
+  // much again in page faults and new threads, more than one download gains (the first pass of an
+  // engine in complex128: 512² with one mode 3.7 ms without, 6.7 with; 256² × 2 modes 2.7 and
+  // 3.4). A program that takes one result, object and probe, does not pay for it.
+  static constexpr int kPlain = 2;
 
   // Whether a download of `bytes` goes through the ring, which this makes if it is wanted and
   // missing. Pinned memory or events that are refused leave the caller its plain copy.
   bool ready(size_t bytes) {
     if (host_) return bytes >= 2 * kPiece;
-    if (bytes < kMin) return false;
+    if (bytes < kMin || large_++ < kPlain) return false;
     if (prepare() == hipSuccess) return true;
     (void)hipGetLastError();  // the next launch's check must not report it
     return false;
@@ -128,6 +133,7 @@ class DownloadRing {
   }
   void* at(int slot) const { return static_cast<char*>(host_) + size_t(slot) * kPiece; }
   void* host_ = nullptr;
+  size_t large_ = 0;  // downloads from kMin on before there was a ring
   hipEvent_t done_[kSlots] = {};
 };
 

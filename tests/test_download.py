@@ -67,11 +67,19 @@ bool whole(DownloadRing& ring, size_t count) {
   return true;
 }
 
+// A ring past the large downloads that go without it.
+struct Used : DownloadRing {
+  Used() {
+    for (int i = 0; i < kPlain; ++i) first |= ready(32 << 20);
+  }
+  bool first = false;
+};
+
 template <typename T>
 int run() {
   const size_t large = 32 << 20, mid = 2 << 20, small = 100000;
   {
-    DownloadRing ring;  // nothing to be had: no ring, no error left, and no second try fails
+    Used ring;  // nothing to be had: no ring, no error left, and no second try fails
     refuse_host = 1;
     CHECK(!ring.ready(large) && last == 0);
     CHECK(!ring.ready(large) && last == 0);
@@ -81,7 +89,9 @@ int run() {
   }
   CHECK(pinned == 0 && events == 0);
   {
-    DownloadRing ring;
+    Used ring;
+    CHECK(!ring.first && pinned == 0 && events == 0);  // one result costs no ring
+    for (int i = 0; i < 5; ++i) CHECK(!ring.ready(mid));
     refuse_event = 3;
     CHECK(!ring.ready(large) && last == 0 && pinned == 0);
     refuse_event = -1;
