@@ -1106,11 +1106,11 @@ class Engine : public EngineBase {
                            tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_,
                            g, tw_.as<cplx<T>>());
-        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+        hipLaunchKernelGGL(k_unramp_mean<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                            gP_.as<cplx<T>>(), (const cplx<T>*)g,
                            (const double2*)offs_.as<double2>(), ord, nb, N, M_,
-                           1.0 / double(n), int(s > 0));
+                           1.0 / double(n), int(s > 0), sum_px());
       });
     }
     run(K_PROBE, [&] {
@@ -1529,12 +1529,12 @@ class Engine : public EngineBase {
         });
       }
       if (up) {
-        const int nblk = (n + REDUCE_PX - 1) / REDUCE_PX;
+        const int nblk = int(reduce_blocks());
         run(K_PROBE, [&] {
           hipLaunchKernelGGL(k_probe_reduce<T>, dim3(nblk, M_ + 1), dim3(REDUCE_THREADS), 0,
                              stream_,
                              pnum_part_.as<cplx<T>>(), pden_part_.as<T>(), nstack * nchunk, n,
-                             M_, gP_.as<cplx<T>>(), pden_.as<T>(), pmaxpart_.as<T>());
+                             M_, gP_.as<cplx<T>>(), pden_.as<T>(), pmaxpart_.as<T>(), sum_px());
         });
       }
       // Polak–Ribière β over both arrays, then the direction; h keeps this cycle's g.
@@ -1748,11 +1748,11 @@ class Engine : public EngineBase {
                                g, tw_.as<cplx<T>>());
             hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0,
                                stream_, g, tw_.as<cplx<T>>());
-            hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+            hipLaunchKernelGGL(k_unramp_mean<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0,
                                stream_, gP_.as<cplx<T>>(), (const cplx<T>*)g,
                                (const double2*)offs_.as<double2>(), ord, nb, N, M_,
-                               1.0 / double(n), int(s > 0));
+                               1.0 / double(n), int(s > 0), sum_px());
           });
         }
       }
@@ -1954,11 +1954,11 @@ class Engine : public EngineBase {
         run(K_PASS_C, [&] { rows(true, K); });
         if (up)
           run(K_PROBE, [&] {
-            hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+            hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0,
                                stream_, gP_.as<cplx<T>>(), (const cplx<T>*)win, N,
                                (const cplx<T>*)q_.as<cplx<T>>(), g, fo_tall_.as<int2>(), ord, nb,
-                               N, M_, T(1), int(s > 0));
+                               N, M_, T(1), int(s > 0), sum_px());
           });
         if (uo)
           run(K_OBJ_UPDATE, [&] {
@@ -3055,10 +3055,10 @@ class Engine : public EngineBase {
       hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_, gg,
                          tw_.as<cplx<T>>());
       // g_P = conj(q)·Σ_b DFT⁻¹(G_b·exp(+2πi f·d_b))
-      hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+      hipLaunchKernelGGL(k_unramp_mean<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                          bh_gP_.as<cplx<T>>(), (const cplx<T>*)gg, offs, ord, nb, N, M_,
-                         1.0 / double(n), 0);
+                         1.0 / double(n), 0, sum_px());
       inverse_planes(bh_gP_.as<cplx<T>>(), M_);
       hipLaunchKernelGGL((k_times_q<T, true>), dim3((n + 255) / 256, M_), dim3(256), 0, stream_,
                          bh_gP_.as<cplx<T>>(), (const cplx<T>*)q_.as<cplx<T>>(), n);
@@ -3196,12 +3196,12 @@ class Engine : public EngineBase {
       });
     }
     run(K_PROBE, [&] {
-      hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+      hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                          bh_gP_.as<cplx<T>>(),
                          fo ? (const cplx<T>*)fo_swin(0) : (const cplx<T>*)slice_obj(0),
                          fo ? N : int(nxo_), (const cplx<T>*)nullptr, (const cplx<T>*)chi,
-                         fo ? fo_tall_.as<int2>() : corner_.as<int2>(), ord, nb, N, M_, T(1), 0);
+                         fo ? fo_tall_.as<int2>() : corner_.as<int2>(), ord, nb, N, M_, T(1), 0, sum_px());
     });
     const int ndots =
         int(std::min<size_t>(kBhDotBlocks, (no + np + THREADS - 1) / THREADS));
@@ -3756,10 +3756,10 @@ class Engine : public EngineBase {
         });
       }
       run(K_PROBE, [&] {
-        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(), (const cplx<T>*)slice_obj(0), int(nxo_), q0,
-                           (const cplx<T>*)chi, corner_.as<int2>(), ord, nb, N, M_, T(1), acc);
+                           (const cplx<T>*)chi, corner_.as<int2>(), ord, nb, N, M_, T(1), acc, sum_px());
       });
     }
     // Not through the ring: its workers compete with the host threads that a torch program's own
@@ -3947,11 +3947,11 @@ class Engine : public EngineBase {
                            tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_, g,
                            tw_.as<cplx<T>>());
-        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+        hipLaunchKernelGGL(k_unramp_mean<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(), (const cplx<T>*)g,
                            (const double2*)offs_.as<double2>(), ord, nb, N, M_,
-                           1.0 / (double(n) * double(nb)));
+                           1.0 / (double(n) * double(nb)), 0, sum_px());
         hipLaunchKernelGGL((k_cols<T, N, true>), dim3(SC::NBLK, M_), dim3(SC::NT), 0, stream_,
                            dPm_.as<cplx<T>>(), tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_rows<T, N, true>), dim3(S::NBLK, M_), dim3(S::NT), 0, stream_,
@@ -3976,13 +3976,13 @@ class Engine : public EngineBase {
       });
     } else {
       run(K_PROBE, [&] {
-        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+        hipLaunchKernelGGL(k_ms_probe_dir<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(),
                            fo ? (const cplx<T>*)fo_swin(0) : (const cplx<T>*)slice_obj(0),
                            fo ? N : int(nxo_), q0, (const cplx<T>*)chi,
                            fo ? fo_tall_.as<int2>() : corner_.as<int2>(), ord, nb, N, M_,
-                           T(1) / T(nb), 0);
+                           T(1) / T(nb), 0, sum_px());
       });
     }
     const int total = int(nprobe_ * n);
@@ -4116,13 +4116,13 @@ class Engine : public EngineBase {
   }
 
   void probe_blend(int tot_chunks, double inertia) {
-    const int nblk = (n + REDUCE_PX - 1) / REDUCE_PX;
+    const int nblk = int(reduce_blocks());
     const int total = int(nprobe_ * n);
     run(K_PROBE, [&] {
       hipLaunchKernelGGL(k_probe_reduce<T>, dim3(nblk, M_ + 1), dim3(REDUCE_THREADS), 0,
                              stream_,
                          pnum_part_.as<cplx<T>>(), pden_part_.as<T>(), tot_chunks, n, M_,
-                         pnum_.as<cplx<T>>(), pden_.as<T>(), pmaxpart_.as<T>());
+                         pnum_.as<cplx<T>>(), pden_.as<T>(), pmaxpart_.as<T>(), sum_px());
       hipLaunchKernelGGL(k_max_reduce<T>, dim3(1), dim3(MAX_THREADS), 0, stream_,
                          pmaxpart_.as<T>(), nblk, pmax2_.as<T>());
       hipLaunchKernelGGL(k_probe_blend<T>, dim3((total + 255) / 256), dim3(256), 0, stream_,
@@ -4222,6 +4222,9 @@ class Engine : public EngineBase {
       });
     });
   }
+  // The slot and chunk sums' pixels per workgroup, and their workgroups per mode.
+  int sum_px() const { return reduce_px((long long)M_ * n); }
+  unsigned reduce_blocks() const { return unsigned((n + sum_px() - 1) / sum_px()); }
   // Workgroups of k_probe_apply and k_probe_mean.
   static unsigned chunk_blocks(int total, int nchunk) {
     const int px = chunk_px(nchunk, THREADS);
@@ -4690,11 +4693,11 @@ class Engine : public EngineBase {
                            tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_cols<T, N, false>), dim3(SC::NBLK, K), dim3(SC::NT), 0, stream_, g,
                            tw_.as<cplx<T>>());
-        hipLaunchKernelGGL(k_unramp_mean<T>, dim3((n + REDUCE_PX - 1) / REDUCE_PX, M_),
+        hipLaunchKernelGGL(k_unramp_mean<T>, dim3(reduce_blocks(), M_),
                            dim3(REDUCE_THREADS), 0, stream_,
                            dPm_.as<cplx<T>>(), (const cplx<T>*)g,
                            (const double2*)offs_.as<double2>(), ord, nb, N, M_,
-                           1.0 / (double(n) * double(nb)));
+                           1.0 / (double(n) * double(nb)), 0, sum_px());
         hipLaunchKernelGGL((k_cols<T, N, true>), dim3(SC::NBLK, M_), dim3(SC::NT), 0, stream_,
                            dPm_.as<cplx<T>>(), tw_.as<cplx<T>>());
         hipLaunchKernelGGL((k_rows<T, N, true>), dim3(S::NBLK, M_), dim3(S::NT), 0, stream_,

@@ -26,8 +26,15 @@
 namespace ptyrs {
 
 constexpr int THREADS = 256;
-// The slot and chunk sums over 64 pixels a workgroup: 16 groups of a wave each.
-constexpr int REDUCE_THREADS = 1024, REDUCE_PX = 64;
+// The slot and chunk sums: a workgroup's REDUCE_THREADS threads take px of the `values` sums
+// (pixels × modes) and share out the slots or chunks over REDUCE_THREADS/px groups, 16 at most and
+// no more than fill the chip once (256 CUs of 2048 threads).
+constexpr int REDUCE_THREADS = 1024, REDUCE_PX = 64, REDUCE_CHIP = 256 * 2048;
+constexpr int reduce_px(long long values) {
+  int px = REDUCE_PX;
+  while (px < REDUCE_THREADS && values * (REDUCE_THREADS / px) > REDUCE_CHIP) px *= 2;
+  return px;
+}
 
 // Elements per thread for a line of n: `pref` where its radix plan exists and the line fits in
 // THREADS_MAX threads, else the first divisor of n that has a plan.
@@ -1875,30 +1882,31 @@ __global__ __launch_bounds__((RowShape<T, N>::NT)) void k_rows_ms(
   for (int e = 0; e < E; ++e) st(row + jl + TL * e, v[e]);
 }
 
-// Sums over a batch's slots per pixel and mode: REDUCE_PX pixels a workgroup of REDUCE_THREADS, 16
-// thread groups taking a contiguous share of the slots each. One thread per pixel left most of the
-// chip idle behind a chain over the slots (128 slots of 128² × 2 modes: 39 µs, 10.6 so; a 50-slot mean of moved spectra 30 µs, 11.6).
-__device__ __forceinline__ int2 slot_share(int g, int nb) {
-  constexpr int NG = REDUCE_THREADS / REDUCE_PX;
-  const int per = (nb + NG - 1) / NG;
+// The share of a batch's slots that group g of ng takes. The groups are whole waves: with g read
+// from the first lane the slots' corners and offsets stay scalar loads.
+__device__ __forceinline__ int2 slot_share(int g, int ng, int nb) {
+  const int per = (nb + ng - 1) / ng;
   const int lo = g * per, hi = lo + per;
   return int2{lo < nb ? lo : nb, hi < nb ? hi : nb};
 }
 
 // The probe direction of slice 0: dP_m = scale·Σ_b conj(O_0[win_b]·q)·χ_0[b·M + m] (Kahan);
 // scale 1/nb for LSQML's frame mean, 1 for a gradient's sum, which `accumulate` adds to dP. Grid
-// (ceil(n/REDUCE_PX), M). ptyrs/src/engine/lsqml.rs:200-229
+// (ceil(n/px), M), px of reduce_px. One thread a pixel left most of the chip idle behind a chain
+// over the slots at 128² (128 slots × 1 mode: 47 µs, 7.7 with 16 groups; 256² × 1 mode 49 and 17
+// with 8); at 512² × 2 modes the pixels alone fill it: 16 groups 162 µs, one 118.
+// ptyrs/src/engine/lsqml.rs:200-229
 template <typename T>
 __global__ __launch_bounds__(REDUCE_THREADS) void k_ms_probe_dir(
     cplx<T>* __restrict__ dP, const cplx<T>* __restrict__ O, int nxo,
     const cplx<T>* __restrict__ q, const cplx<T>* __restrict__ chi,
     const int2* __restrict__ corner, const int* __restrict__ order, int nb, int N, int M, T scale,
-    int accumulate) {
+    int accumulate, int px) {
   __shared__ T part[4 * REDUCE_THREADS];
   const int n = N * N;
-  const int j = blockIdx.x * REDUCE_PX + threadIdx.x % REDUCE_PX;
+  const int tid = threadIdx.x, j = blockIdx.x * px + tid % px;
   const int m = blockIdx.y, y = j / N, x = j % N;
-  const int2 sh = slot_share(threadIdx.x / REDUCE_PX, nb);
+  const int2 sh = slot_share(__builtin_amdgcn_readfirstlane(tid / px), REDUCE_THREADS / px, nb);
   kahan<T> sr, si;
   if (j < n) {
     const cplx<T> qj = q ? ld(q + j) : cplx<T>{T(1), T(0)};
@@ -1910,8 +1918,8 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_ms_probe_dir(
       si.add(g.y);
     }
   }
-  merge_px<T, REDUCE_THREADS>(sr, si, REDUCE_PX, part);
-  if (threadIdx.x >= REDUCE_PX || j >= n) return;
+  if (px < REDUCE_THREADS) merge_px<T, REDUCE_THREADS>(sr, si, px, part);
+  if (tid >= px || j >= n) return;
   cplx<T> v = cplx<T>{sr.s, si.s} * scale;
   if (accumulate) v = v + ld(dP + (size_t)m * n + j);
   st(dP + (size_t)m * n + j, v);
@@ -2033,18 +2041,18 @@ __global__ void k_ramp_planes(cplx<T>* out, const cplx<T>* spec, const double2* 
 }
 
 // The frame mean of spectra moved back: out[m] = scale·Σ_b G[b·M + m]·exp(+2πi f·d_b) (Kahan, the
-// slots shared out as in k_ms_probe_dir). Grid (ceil(n/REDUCE_PX), M).
+// slots shared out as in k_ms_probe_dir). Grid (ceil(n/px), M).
 // ptyrs/src/engine/lsqml.rs:207-229
 // With `accumulate` the result is added to out (a sum over stacks, in stack order).
 template <typename T>
 __global__ __launch_bounds__(REDUCE_THREADS) void k_unramp_mean(
     cplx<T>* __restrict__ out, const cplx<T>* __restrict__ G, const double2* __restrict__ offs,
-    const int* __restrict__ order, int nb, int N, int M, double scale, int accumulate = 0) {
+    const int* __restrict__ order, int nb, int N, int M, double scale, int accumulate, int px) {
   __shared__ T part[4 * REDUCE_THREADS];
   const int n = N * N;
-  const int j = blockIdx.x * REDUCE_PX + threadIdx.x % REDUCE_PX;
+  const int tid = threadIdx.x, j = blockIdx.x * px + tid % px;
   const int m = blockIdx.y;
-  const int2 sh = slot_share(threadIdx.x / REDUCE_PX, nb);
+  const int2 sh = slot_share(__builtin_amdgcn_readfirstlane(tid / px), REDUCE_THREADS / px, nb);
   kahan<T> sr, si;
   if (j < n) {
     const double fy = dft_freq(j / N, N), fx = dft_freq(j % N, N);
@@ -2057,8 +2065,8 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_unramp_mean(
       si.add(T(double(v.x) * s + double(v.y) * c));
     }
   }
-  merge_px<T, REDUCE_THREADS>(sr, si, REDUCE_PX, part);
-  if (threadIdx.x >= REDUCE_PX || j >= n) return;
+  if (px < REDUCE_THREADS) merge_px<T, REDUCE_THREADS>(sr, si, px, part);
+  if (tid >= px || j >= n) return;
   cplx<T> r{T(double(sr.s) * scale), T(double(si.s) * scale)};
   if (accumulate) r = r + ld(out + (size_t)m * n + j);
   st(out + (size_t)m * n + j, r);
@@ -2439,43 +2447,41 @@ __global__ __launch_bounds__(THREADS) void k_probe_sums(
 }
 
 // Sums the probe partials over chunks (Kahan) into num[M][n] and den[n], and writes the per
-// workgroup max of den for the regulariser. Grid (ceil(n/64), M + 1) of REDUCE_THREADS: 64
-// pixels of one mode's num (or, y = M, of den), the chunks shared out over 16 thread groups.
-// One thread per pixel walking every chunk of every mode left 3/4 of the CUs idle at 128² and
-// took 252 µs for 256 chunks of 2 modes; this takes 21.
+// workgroup max of den for the regulariser. Grid (ceil(n/px), M + 1) of REDUCE_THREADS, px of
+// reduce_px: px pixels of one mode's num (or, y = M, of den), the chunks shared out over the
+// thread groups. One thread per pixel walking every chunk of every mode left 3/4 of the CUs idle
+// at 128² and took 252 µs for 256 chunks of 2 modes; this takes 12; 12 chunks
+// at 512² × 2 modes took 62 µs with 16 groups and take 13 with the one of reduce_px.
 template <typename T>
 __global__ __launch_bounds__(REDUCE_THREADS) void k_probe_reduce(
     const cplx<T>* __restrict__ num_part, const T* __restrict__ den_part, int nchunk, int n, int M,
-    cplx<T>* __restrict__ num, T* __restrict__ den, T* __restrict__ maxpart) {
-  constexpr int BT = REDUCE_THREADS, NG = BT / REDUCE_PX;
+    cplx<T>* __restrict__ num, T* __restrict__ den, T* __restrict__ maxpart, int px) {
+  constexpr int BT = REDUCE_THREADS;
   __shared__ T part[4 * BT];
-  const int tid = threadIdx.x, p = tid % REDUCE_PX, g = tid / REDUCE_PX, m = blockIdx.y;
-  const int i = blockIdx.x * REDUCE_PX + p;
+  const int tid = threadIdx.x, p = tid % px, g = tid / px, ng = BT / px, m = blockIdx.y;
+  const int i = blockIdx.x * px + p;
   if (m < M) {
     const int e = m * n + i;  // the element of a chunk's [M][n] planes; past n it is not summed
     kahan<T> sr, si;
-    if (chunk_sum<T, BT>(num_part, nchunk, M * n, i < n ? e : M * n, REDUCE_PX, part, sr, si))
+    if (chunk_sum<T, BT>(num_part, nchunk, M * n, i < n ? e : M * n, px, part, sr, si))
       st(num + e, cplx<T>{sr.s, si.s});
     return;
   }
-  const int per = (nchunk + NG - 1) / NG;
-  const int c1 = (g + 1) * per < nchunk ? (g + 1) * per : nchunk;
+  const int2 sh = slot_share(g, ng, nchunk);
   kahan<T> d;
   if (i < n)
-    for (int c = g * per; c < c1; ++c) d.add(den_part[(size_t)c * n + i]);
+    for (int c = sh.x; c < sh.y; ++c) d.add(den_part[(size_t)c * n + i]);
   part[tid] = d.s;
   part[BT + tid] = d.c;
   __syncthreads();
-  if (g > 0) return;
-  for (int k = 1; k < NG; ++k) d.merge(part[k * REDUCE_PX + p], part[BT + k * REDUCE_PX + p]);
   T mx = 0;
-  if (i < n) {
+  if (g == 0 && i < n) {
+    for (int k = 1; k < ng; ++k) d.merge(part[k * px + p], part[BT + k * px + p]);
     den[i] = d.s;
     mx = d.s;
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mx = MaxOp()(mx, __shfl_xor(mx, off, 64));
-  if (p == 0) maxpart[blockIdx.x] = mx;
+  const T r = block_reduce<BT>(mx, part + 2 * BT, MaxOp());
+  if (tid == 0) maxpart[blockIdx.x] = r;
 }
 
 // PyNX blend of the probe: P = (num + reg·P)/max(den + reg, 1e-12), reg = inertia·max(den);
