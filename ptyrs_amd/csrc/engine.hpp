@@ -1522,7 +1522,7 @@ class Engine : public EngineBase {
       }
       if (uo) {
         run(K_OBJ_UPDATE, [&] {
-          obj_dir(gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
+          obj_dir(int(nframe_), gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
                   corner_.as<int2>(), iota_.as<int>(), list_all_.as<int>(),
                   count_all_.as<int>(), int(nframe_), int(nyo_), int(nxo_), ntx_,
                   (const T*)nullptr, (const T*)nullptr, 0, nullptr, 0, 0, true);
@@ -1768,7 +1768,7 @@ class Engine : public EngineBase {
       }
       if (uo) {
         run(K_OBJ_UPDATE, [&] {
-          obj_dir(gO_.as<cplx<T>>(), (const cplx<T>*)wall, carried_.as<cplx<T>>(),
+          obj_dir(int(nframe_), gO_.as<cplx<T>>(), (const cplx<T>*)wall, carried_.as<cplx<T>>(),
                              N, M_, corner_.as<int2>(), iota_.as<int>(), list_all_.as<int>(),
                              count_all_.as<int>(), int(nframe_), int(nyo_), int(nxo_), ntx_,
                              (const T*)nullptr, (const T*)nullptr, 1, (const cplx<T>*)nullptr,
@@ -3041,7 +3041,7 @@ class Engine : public EngineBase {
                          chunk, 0, dP_.as<cplx<T>>(), tw_.as<cplx<T>>(), 0);
     });
     run(K_OBJ_DIR, [&] {
-      obj_dir(bh_gO_.as<cplx<T>>(), (const cplx<T>*)w, psi_.as<cplx<T>>(), N, M_,
+      obj_dir(nb, bh_gO_.as<cplx<T>>(), (const cplx<T>*)w, psi_.as<cplx<T>>(), N, M_,
                          corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                          int(nyo_), int(nxo_), ntx_, (const T*)nullptr, (const T*)nullptr, 1);
     });
@@ -3184,7 +3184,7 @@ class Engine : public EngineBase {
           fo_add_placed<AS_PLAIN>(bh_gO_.as<cplx<T>>() + s * no1, 1.0);
           return;
         }
-        obj_dir(bh_gO_.as<cplx<T>>() + s * no1, in.first, (const cplx<T>*)chi, N, M_,
+        obj_dir(nb, bh_gO_.as<cplx<T>>() + s * no1, in.first, (const cplx<T>*)chi, N, M_,
                            corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                            int(nyo_), int(nxo_), ntx_, (const T*)nullptr, (const T*)nullptr,
                            in.second, qs, 0);
@@ -3520,7 +3520,7 @@ class Engine : public EngineBase {
                          chunk, 1, dP_.as<cplx<T>>(), tw_.as<cplx<T>>(), 0);
     });
     run(K_OBJ_DIR, [&] {
-      obj_dir(bh_gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
+      obj_dir(nb, bh_gO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), psi_.as<cplx<T>>(), N, M_,
                          corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_),
                          int(nyo_), int(nxo_), ntx_, (const T*)nullptr, (const T*)nullptr);
     });
@@ -3594,7 +3594,7 @@ class Engine : public EngineBase {
                            (const cplx<T>*)nullptr);
       });
       run(K_OTHER, [&] {
-        split_tiles([&](auto sp) {
+        split_tiles(nb, kSplitGather, [&](auto sp) {
           constexpr int SP = decltype(sp)::value;
           hipLaunchKernelGGL((k_illumination<T, SP>), dim3(nt), dim3(THREADS * SP), 0, stream_,
                            illum_.as<T>(), P_.as<cplx<T>>(), N, M_, corner_.as<int2>(), ord,
@@ -3660,7 +3660,7 @@ class Engine : public EngineBase {
     pass_c_sum<true>(ord, nb, chunk, linear ? (const T*)afar_tmp_.as<T>() : nullptr, true,
                      csum_.as<cplx<T>>(), false, dP_.as<cplx<T>>(), nullptr);
     run(K_OBJ_DIR, [&] {
-      obj_dir(dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
+      obj_dir(nb, dO_.as<cplx<T>>(), Wt_.as<cplx<T>>(), csum_.as<cplx<T>>(), N, M_,
               corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(), int(cap_), int(nyo_),
               int(nxo_), ntx_, pre_.as<T>(), floor_.as<T>(), 0, nullptr, 0, 0, true);
     });
@@ -3744,7 +3744,7 @@ class Engine : public EngineBase {
         const auto in = wave(s, wv);
         const cplx<T>* qs = s + 1 == S ? q_.as<cplx<T>>() : nullptr;
         run(K_OBJ_UPDATE, [&] {
-          obj_dir(slice_dir(s), in.first, (const cplx<T>*)chi, N, M_,
+          obj_dir(nb, slice_dir(s), in.first, (const cplx<T>*)chi, N, M_,
                              corner_.as<int2>(), ord, list_.as<int>(), lcount_.as<int>(),
                              int(cap_), int(nyo_), int(nxo_), ntx_, (const T*)nullptr,
                              (const T*)nullptr, in.second, qs, 0, acc);
@@ -3907,7 +3907,7 @@ class Engine : public EngineBase {
                              (const T*)floor_.as<T>(), nol);
           return;
         }
-        obj_dir(slice_dir(s), in.first, (const cplx<T>*)chi, N, M_, corner_.as<int2>(),
+        obj_dir(nb, slice_dir(s), in.first, (const cplx<T>*)chi, N, M_, corner_.as<int2>(),
                            ord, list_.as<int>(), lcount_.as<int>(), int(cap_), int(nyo_),
                            int(nxo_), ntx_, pre_.as<T>(), floor_.as<T>(), in.second, qs, qf);
       });
@@ -4183,10 +4183,10 @@ class Engine : public EngineBase {
     return M_ <= kBWideModes ? BShape<T, N, 1>::NBLK : BShape<T, N, kMaxModes>::NBLK;
   }
   int ntiles() const { return ntx_ * nty_; }
-  // The tile kernels' split (SP of them share a tile's views; kernels.hpp): by the tile count.
+  // The tile kernels' split: SP thread groups share a tile's views (kernels.hpp).
   template <typename F>
-  void split_tiles(F&& f) {
-    if (ntiles() < kSplitTiles)
+  void split_tiles(int views, int cost, F&& f) {
+    if (tile_split(ntiles(), views, cost))
       f(std::integral_constant<int, 4>{});
     else
       f(std::integral_constant<int, 1>{});
@@ -4233,7 +4233,8 @@ class Engine : public EngineBase {
   void bin_tiles(const int2* corner, const int* ord, int nb, int side, int ntx, int cap, int* list,
                  int* count, const T* W2, int M, int nyo, int nxo, T* D, T* tilemax,
                  const cplx<T>* Wv) {
-    split_tiles([&](auto sp) {
+    const int cost = W2 || Wv ? (M > 1 ? kSplitOverlaps : kSplitOverlap) : kSplitNever;
+    split_tiles(nb, cost, [&](auto sp) {
       mode_chunk(false, [&](auto mm) {
         constexpr int SP = decltype(sp)::value, VW = decltype(mm)::value;
         if constexpr (VW > 0)
@@ -4243,12 +4244,12 @@ class Engine : public EngineBase {
       });
     });
   }
-  void obj_dir(cplx<T>* dO, const cplx<T>* Wt, const cplx<T>* chi, int side, int M,
+  void obj_dir(int views, cplx<T>* dO, const cplx<T>* Wt, const cplx<T>* chi, int side, int M,
                const int2* corner, const int* ord, const int* list, const int* count, int cap,
                int nyo, int nxo, int ntx, const T* pre, const T* floor, int per_view = 0,
                const cplx<T>* q = nullptr, int q_frame = 0, int accumulate = 0,
                bool summed = false) {
-    split_tiles([&](auto sp) {
+    split_tiles(views, kSplitGather, [&](auto sp) {
       mode_chunk(summed, [&](auto mm) {
         constexpr int SP = decltype(sp)::value, MM = decltype(mm)::value;
         hipLaunchKernelGGL((k_lsqml_obj_dir<T, SP, MM>), dim3(ntiles()), dim3(THREADS * SP), 0,
@@ -4273,7 +4274,8 @@ class Engine : public EngineBase {
                  const int2* corner, const int* ord, const int* list, const int* count, int cap,
                  int nyo, int nxo, int ntx, const T* nmax, T inertia, int w_view = 0,
                  bool summed = false) {
-    split_tiles([&](auto sp) {
+    // Every landed frame is over the blend's tiles.
+    split_tiles(int(nframe_), kSplitGather, [&](auto sp) {
       mode_chunk(summed, [&](auto mm) {
         constexpr int SP = decltype(sp)::value, MM = decltype(mm)::value;
         hipLaunchKernelGGL((k_obj_blend<T, H, SP, MM>), dim3(ntiles()), dim3(THREADS * SP), 0,
@@ -4593,7 +4595,7 @@ class Engine : public EngineBase {
     if (upd_obj && upd_probe) {
       const int total = int(nprobe_ * n);
       run(K_OBJ_UPDATE, [&] {
-        split_tiles([&](auto sp) {
+        split_tiles(nb, kSplitGather, [&](auto sp) {
           constexpr int SP = decltype(sp)::value, BT = THREADS * SP;
           const int px = chunk_px(nchunk, BT);
           hipLaunchKernelGGL((k_rpie_updates<T, SP>), dim3(nt + (total + px - 1) / px), dim3(BT), 0,
@@ -4609,7 +4611,7 @@ class Engine : public EngineBase {
     }
     if (upd_obj) {
       run(K_OBJ_UPDATE, [&] {
-        split_tiles([&](auto sp) {
+        split_tiles(nb, kSplitGather, [&](auto sp) {
           constexpr int SP = decltype(sp)::value;
           hipLaunchKernelGGL((k_obj_update_rpie_sum<T, SP>), dim3(nt), dim3(THREADS * SP), 0, stream_,
                            O_.as<cplx<T>>(), (const cplx<T>*)psi_.as<cplx<T>>(), N, M_,
@@ -4674,7 +4676,7 @@ class Engine : public EngineBase {
     if (pos_refine_) position_sums(0, W, nullptr, 0, ord, nb, chi0);
     if (upd_obj) {
       run(K_OBJ_UPDATE, [&] {
-        split_tiles([&](auto sp) {
+        split_tiles(nb, kSplitGather, [&](auto sp) {
           constexpr int SP = decltype(sp)::value;
           hipLaunchKernelGGL((k_obj_update_rpie_sum<T, SP>), dim3(nt), dim3(THREADS * SP), 0, stream_,
                            O_.as<cplx<T>>(), (const cplx<T>*)psi_.as<cplx<T>>(), N, M_,

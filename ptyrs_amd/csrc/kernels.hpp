@@ -1004,15 +1004,32 @@ __global__ __launch_bounds__(THREADS) void k_probe_apply(
 // ---- object tiles --------------------------------------------------------------------------------
 // Object tiles of 64×4 pixels. A tile's workgroup has SP groups of THREADS threads, each with
 // one thread per pixel; a round stages up to THREADS of the tile's views in LDS, group g takes
-// the g-th contiguous share of them, and the groups' sums meet in LDS in group order. A pixel's
-// views are a serial chain of loads and compensated adds, so with few tiles the chip idles and
-// the chain is the time: SP = 4 below kSplitTiles tiles (tile_split), 1 above, where the tiles
-// alone fill it and the split would only add its combination. SP = 1 → 4, complex64: rPIE's
-// overlaps 22.8 → 10.8 µs and updates 31 → 11.4 (126 tiles, 64² frames, 100 views), LSQML's object
-// direction 89 → 25 µs (400 tiles, 128 views of 128² × 2 modes); at 5076 tiles SP = 1 runs.
+// the g-th contiguous share of them, and the groups' sums meet in LDS in group order.
 constexpr int TILE_X = 64, TILE_Y = 4;
 static_assert(TILE_X * TILE_Y == THREADS, "a tile has one thread per pixel");
-constexpr int kSplitTiles = 2048;
+
+// Whether four groups (SP = 4) share a tile's views, else SP = 1. A pixel's views are a serial
+// chain of loads and compensated adds: with few tiles the chip idles and the chain is the time.
+// But a split workgroup takes half a CU, so 512 tiles are a round of them where 2048 are one of
+// the unsplit, and each pays its staging, barriers and combination. The views from which the split
+// gains grow about as the square of the rounds: `cost` is the views at one round, least the fewest
+// at any tile count. Measured in complex64 (µs of a launch, unsplit | split):
+//   gathers (object updates, directions, blends, illumination): rPIE's update at 130 tiles 2 views
+//     4.7 | 4.7, 32 views 11.0 | 5.5; 700 tiles 8 views 7.4 | 7.8, 16 views 12.0 | 9.6; 1300 tiles
+//     16 views 10.3 | 13.6, 32 views 15.8 | 15.2; 1900 tiles 64 views 20.8 | 21.3, 128 views
+//     33.7 | 26.9. LSQML's direction at 400 tiles, 128 views of 2 modes 89 | 25.
+//   overlaps of one mode: 130 tiles 8 views 5.2 | 5.2; 700 tiles 16 views 8.8 | 9.2, 24 views
+//     10.9 | 9.4; 1000 tiles 32 views 12.4 | 12.2; 1900 tiles 128 views 21.7 | 24.0
+//   of four, whose sums the groups exchange mode by mode: 330 tiles 16 views 9.2 | 8.3; 700 tiles
+//     32 views 14.8 | 15.5; 1300 tiles 32 views 13.4 | 23.1; 1900 tiles 128 views 26.0 | 45.3
+//   lists alone: 330 to 1900 tiles, 1 to 32 views, 4 | 5 to 13
+constexpr int kSplitTiles = 2048, kSplitLeast = 4;
+constexpr int kSplitGather = 5, kSplitOverlap = 10, kSplitOverlaps = 20, kSplitNever = 0;
+constexpr bool tile_split(long long tiles, long long views, int cost) {
+  constexpr long long round = 512;
+  return cost != kSplitNever && tiles < kSplitTiles && views >= kSplitLeast &&
+         views * round * round >= cost * tiles * tiles;
+}
 
 // Views [lo, hi) of a round of k staged views that group g of SP takes.
 template <int SP>

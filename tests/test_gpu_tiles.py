@@ -1,7 +1,8 @@
 """The object tile kernels and the probe sums at the edges of their splits, against the FP64
-oracle in complex128: an object of more tiles than the split takes and of fewer, tiles with more
-views than one round stages (256), one mode and an odd number, and chunk counts of the probe
-sums on both sides of their own split. 1e-9 is the complex128 bound of the other parity tests:
+oracle in complex128: an object of more tiles than the split takes and of fewer, batches of more
+and fewer views than it needs there, one where the gathers are split and the overlaps are not, tiles
+with more views than one round stages (256), one mode and an odd number, and chunk counts of the
+probe sums on both sides of their own split. 1e-9 is the complex128 bound of the other parity tests:
 the splits only regroup sums of at most 300 terms (300·2^-53 = 3e-14)."""
 
 import math
@@ -16,9 +17,13 @@ from ptyrs_amd import sim
 
 pytestmark = pytest.mark.gpu
 
-# frame side, modes, frames, object (rows, columns): 40 tiles of 300 views each; 2100 tiles,
-# above the split, the last column and row of tiles ragged.
-CASES = [(16, 1, 300, (40, 40)), (16, 3, 20, (40, 72)), (32, 3, 12, (1002, 500))]
+# frame side, modes, frames, object (rows, columns): 10 tiles of 300 views each; 20 tiles; 1000
+# tiles, whose gathers split from 20 views on and overlaps from 77; more tiles than are split, the
+# last column and row of them ragged.
+CASES = [(16, 1, 300, (40, 40)), (16, 3, 20, (40, 72)), (32, 3, 24, (500, 500)),
+         (32, 3, 12, (1042, 500))]
+TILES = [math.ceil(c[3][0] / 4) * math.ceil(c[3][1] / 64) for c in CASES]
+assert TILES == [10, 20, 1000, 2088]
 
 
 def scan(case):
@@ -40,6 +45,7 @@ def scan(case):
 
 @pytest.mark.parametrize("case", CASES)
 @pytest.mark.parametrize("name,kw", [("rpie", dict(batch_size=300)), ("rpie", dict(batch_size=7)),
+                                     ("rpie", dict(batch_size=3)),
                                      ("ap", dict(probe_inertia=0.001)),
                                      ("ml", dict(update_probe=True))])
 def test_tiles(case, name, kw):
