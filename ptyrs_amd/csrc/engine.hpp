@@ -506,8 +506,8 @@ class Engine : public EngineBase {
     const size_t cap = std::min(p.batch_size, nframe_);
     ensure_workspace(cap, nepoch);
     if (full_object()) fo_ensure(cap_);
-    if (!pos_on_ && !full_object() && frame_path())
-      dP_.ensure(sizeof(cplx<T>) * cap_ * M_ * n);  // a slot a chunk
+    if (!pos_on_ && !full_object() && frame_path(1))
+      dP_.ensure(sizeof(cplx<T>) * std::min(cap, kFrameSlots) * M_ * n);  // a slot a chunk
     if (pos_on_ && !full_object()) {
       // Under offsets pass C leaves one probe direction per frame, moved back and averaged.
       dP_.ensure(sizeof(cplx<T>) * cap_ * M_ * n);
@@ -4521,10 +4521,15 @@ class Engine : public EngineBase {
     due.clear();
   }
 
-  // One rPIE batch (ptyrs/src/engine/ptycho.rs:900-1086) from the batch-start object and probe.
   // Whether rPIE's batches run k_rpie_frame, a frame a workgroup (frame.hpp): one mode, and one
   // DFT to the detector (the angular spectrum takes two).
-  bool frame_path() const { return whole_frame<T, N>() && M_ == 1 && !angular_; }
+  // Each slot leaves a probe direction of its own: up to kFrameSlots of them (128 MB at 64², where
+  // batches of 4096 take 0.99 ms a pass of two and the stack's passes, with a few hundred chunks'
+  // directions, 1.51), so that larger batches hold no more than the stack.
+  static constexpr size_t kFrameSlots = 4096;
+  bool frame_path(size_t nb) const {
+    return whole_frame<T, N>() && M_ == 1 && !angular_ && nb <= kFrameSlots;
+  }
   void rpie_frames(const ptyrs_rpie_params& p, const int* ord, int nb) {
     if constexpr (whole_frame<T, N>()) {
       run(K_PASS_C, [&] {
@@ -4539,6 +4544,7 @@ class Engine : public EngineBase {
       });
     }
   }
+  // One rPIE batch (ptyrs/src/engine/ptycho.rs:900-1086) from the batch-start object and probe.
   void rpie_batch(const ptyrs_rpie_params& p, const int* ord, int nb) {
     if (full_object()) {
       rpie_batch_sampled(p, ord, nb);
@@ -4552,7 +4558,7 @@ class Engine : public EngineBase {
     const int nt = ntiles();
     // Pass A's launch takes the tiles' max with it where its grid has room for the row.
     const bool fold = upd_obj && size_t(nb) * M_ < 65535;
-    const bool frames = frame_path();
+    const bool frames = frame_path(size_t(nb));
     if (upd_obj) {
       // W2_ holds |W_m|² of the batch-start probe terms (rpie_begin, then each batch's
       // k_rpie_updates; without probe updates the probe does not change).
