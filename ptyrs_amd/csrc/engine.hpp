@@ -2900,7 +2900,7 @@ class Engine : public EngineBase {
   DownloadRing ring_;
   void download_complex(const DevBuf& d, double* out, size_t count) {
     if (ring_.ready(sizeof(cplx<T>) * count)) {
-      PTYRS_HIP(ring_.run(device_, stream_, d.as<const cplx<T>>(), count, out));
+      PTYRS_HIP(ring_.run(stream_, d.as<const cplx<T>>(), count, out));
       return;
     }
     download_plain(d, out, count);
@@ -3762,9 +3762,9 @@ class Engine : public EngineBase {
                            (const cplx<T>*)chi, corner_.as<int2>(), ord, nb, N, M_, T(1), acc, sum_px());
       });
     }
-    // Not through the ring: its workers compete with the host threads that a torch program's own
-    // conversions around this call keep busy (a 10 MB object gradient: 1000 frames of 256², 9.9 ms
-    // a call with the ring and 8.2 without; three slices at 128², 12.7 and 9.1).
+    // Not through the ring: beside the host threads that a torch program's own conversions around
+    // this call keep busy, worker threads cost more than they gave (a 10 MB object gradient: 1000
+    // frames of 256², 9.9 ms a call with them and 8.2 without; three slices at 128², 12.7 and 9.1).
     download_plain(dO_, og, S * no);
     download_plain(dPm_, pg, nprobe_ * n);
     flush_timing();

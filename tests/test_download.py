@@ -1,5 +1,6 @@
 """The state downloads' ring (csrc/download.hpp) on the host: compiled here against a stand-in of
-the few runtime calls it makes, whose allocations can be refused."""
+the few runtime calls it makes, whose allocations can be refused and whose copies can fail; alone,
+and several rings at once on the shared helpers."""
 
 import shutil
 import subprocess
@@ -8,14 +9,20 @@ from conftest import ROOT
 
 RUNTIME = r"""
 #pragma once
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <thread>
+#include <vector>
 using hipError_t = int;
 using hipStream_t = void*;
 using hipEvent_t = void*;
 constexpr int hipSuccess = 0, hipErrorOutOfMemory = 2;
 constexpr int hipEventDisableTiming = 2, hipHostMallocDefault = 0, hipMemcpyDeviceToHost = 2;
 inline int refuse_host = 0, refuse_event = -1, last = 0, events = 0, pinned = 0;
+inline int copies_left = -1;  // copies until one fails
+inline std::thread::id caller;
+inline std::atomic<bool> others{false};  // a runtime call from another thread than the caller's
 inline hipError_t hipGetLastError() { int e = last; last = 0; return e; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   if (refuse_event >= 0 && events >= refuse_event) return last = hipErrorOutOfMemory;
@@ -31,11 +38,16 @@ inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   return hipSuccess;
 }
 inline hipError_t hipHostFree(void* p) { --pinned; std::free(p); return hipSuccess; }
-inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventSynchronize(hipEvent_t) {
+  if (std::this_thread::get_id() != caller) others = true;
+  return hipSuccess;
+}
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
+  if (std::this_thread::get_id() != caller) others = true;
+  if (copies_left == 0) return hipErrorOutOfMemory;
+  if (copies_left > 0) --copies_left;
   std::memcpy(d, s, n);
   return hipSuccess;
 }
@@ -61,25 +73,17 @@ bool whole(DownloadRing& ring, size_t count) {
   std::vector<cplx<T>> src(count);
   for (size_t i = 0; i < count; ++i) src[i] = {T(i), T(-0.5 * double(i))};
   std::vector<double> out(2 * count, 1e300);
-  if (ring.run(0, nullptr, src.data(), count, out.data()) != hipSuccess) return false;
+  if (ring.run(nullptr, src.data(), count, out.data()) != hipSuccess) return false;
   for (size_t i = 0; i < count; ++i)
     if (out[2 * i] != double(src[i].x) || out[2 * i + 1] != double(src[i].y)) return false;
   return true;
 }
 
-// A ring past the large downloads that go without it.
-struct Used : DownloadRing {
-  Used() {
-    for (int i = 0; i < kPlain; ++i) first |= ready(32 << 20);
-  }
-  bool first = false;
-};
-
 template <typename T>
 int run() {
   const size_t large = 32 << 20, mid = 2 << 20, small = 100000;
   {
-    Used ring;  // nothing to be had: no ring, no error left, and no second try fails
+    DownloadRing ring;  // nothing to be had: no ring, no error left, and no second try fails
     refuse_host = 1;
     CHECK(!ring.ready(large) && last == 0);
     CHECK(!ring.ready(large) && last == 0);
@@ -89,9 +93,8 @@ int run() {
   }
   CHECK(pinned == 0 && events == 0);
   {
-    Used ring;
-    CHECK(!ring.first && pinned == 0 && events == 0);  // one result costs no ring
-    for (int i = 0; i < 5; ++i) CHECK(!ring.ready(mid));
+    DownloadRing ring;
+    CHECK(!ring.ready(mid) && events == 0);
     refuse_event = 3;
     CHECK(!ring.ready(large) && last == 0 && pinned == 0);
     refuse_event = -1;
@@ -99,13 +102,40 @@ int run() {
     const size_t piece = DownloadRing::kPiece / sizeof(cplx<T>);
     for (size_t count : {size_t(1), piece, piece + 1, 2 * piece, 8 * piece - 1, 17 * piece + 3,
                          40 * piece})
-      CHECK(whole<T>(ring, count));
+      for (int i = 0; i < 5; ++i) CHECK(whole<T>(ring, count));
+    // A copy that fails ends the download with its error, and the ring serves the next one.
+    std::vector<cplx<T>> src(40 * piece);
+    std::vector<double> out(2 * src.size());
+    for (int k : {0, 1, 7, 8, 13, 39}) {
+      copies_left = k;
+      CHECK(ring.run(nullptr, src.data(), src.size(), out.data()) == hipErrorOutOfMemory);
+      copies_left = -1;
+      CHECK(whole<T>(ring, src.size()));
+    }
   }
   CHECK(pinned == 0 && events == 0);
+  CHECK(!others);  // the helpers only widen
+  {  // several engines' rings at once, sharing the helpers
+    std::atomic<int> bad{0};
+    std::vector<std::thread> threads;
+    std::vector<DownloadRing> rings(6);
+    for (auto& r : rings) CHECK(r.ready(large));
+    for (auto& r : rings)
+      threads.emplace_back([&] {
+        for (int i = 0; i < 10; ++i) bad += !whole<T>(r, 700000);
+      });
+    for (auto& t : threads) t.join();
+    CHECK(bad == 0);
+  }
   return 0;
 }
 
-int main() { return run<float>() || run<double>(); }
+int main() {
+  caller = std::this_thread::get_id();
+  if (run<float>()) return 1;
+  others = false;
+  return run<double>();
+}
 """
 
 

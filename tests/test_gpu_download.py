@@ -1,7 +1,7 @@
 """The state comes back exactly as it was set, at array sizes around the download's pieces: below
-its ring, a piece short of and past its first thread, a ragged last piece, several pieces per
-worker. Objects are read often enough for the ring to be made by them (from 4 MB on), and the
-probe of four modes of 256² (2 MB in complex64, 4 in complex128) goes through it after them."""
+its ring, a piece short of and past its first helper, a ragged last piece, several pieces per
+thread. Each state is read several times; the ring is made by an object of at least 4 MB, and the
+probe of four modes of 256² (2 MB in complex64, 4 in complex128) goes through it after that."""
 
 import numpy as np
 import pytest
